@@ -64,6 +64,7 @@ TILE_I = (256, 512, 1024)            # netra_moe_down_tile_i<I>_gfx950
 ROWS_I = (256, 512)                  # netra_moe_down_rows_i<I>_gfx950 (block rows x runs of column groups)
 DOWN_ROWS_ITEMS = 1024               # down_rows: fewer column groups per item until about this many items
 TILE_GU_WAVES = 4                    # waves of netra_moe_gate_up_tile_h<H>_gfx950 (its launch bound)
+SPLIT_HI = ((2048, 512),)            # netra_moe_gate_up_split_h<H>_{tiles|rows}_gfx950
 LDS_GU_H = (512, 1024, 2048)         # netra_moe_gate_up_lds_h<H>_gfx950: 128-row pairs, LDS operand ring
 # Stream kernel grids (measured at T=64 on one MI355X): gate/up fills the chip
 # once, 256 CUs x 4 SIMDs x 2 resident waves (NK_GATE_UP_WAVES_PER_EU) / 8
@@ -136,6 +137,40 @@ def xcd_grid(items: int) -> int:
     """Workgroups for an XCD-major item assignment (nktile::xcd_item): a
     multiple of 8 covering every item."""
     return (items + 7) // 8 * 8
+
+
+SPLIT_GRID = 256                     # one workgroup per CU
+# Rows per routed expert (T K / E) up to which gate/up is the split kernel.
+# Gate/up times, µs, the path's other kernel / split: T = 80
+# (2.5 rows) 88.1 / 82.2, 192 (6) 115.3 / 98, 400 (12.5) 110.8 / 96.3; with
+# Zipf-skewed routing T = 192 52.1 / 45.4, 400 46.8 / 42.8, 512 (16) 46.0 /
+# 53.0 (uniform at 512: 111 / 96). T = 65 84.3 / 83.6.
+SPLIT_MAX_ROWS = 13
+
+
+def split_gate_up(cfg: MoEConfig, path: str) -> bool:
+    """Whether the stream or tile path's gate/up is the split kernel."""
+    return (path in ("stream", "tile") and (cfg.H, cfg.I) in SPLIT_HI and cfg.T * cfg.H < 1 << 31
+            and cfg.T * cfg.K <= SPLIT_MAX_ROWS * cfg.E and cfg.cap_blocks < 1 << 16)
+
+
+def split_lds_bytes() -> int:
+    """Static LDS of the split gate/up: two split-sum buffers of four row
+    tiles, a 128-column block of h, the chunk table."""
+    return 2 * 8 * 2 * 4 * 1024 + 64 * 136 * 2 + 4 * (2 * 513 + 1) + 20
+
+
+def _split_gate_up(cfg: MoEConfig, path: str) -> dict:
+    u = lambda v: ("u32", int(v))  # noqa: E731
+    routing = ["sorted_ids", "expert_counts"]
+    return dict(name="moe.gate_up",
+                symbol=f"netra_moe_gate_up_split_h{cfg.H}_{'tiles' if path == 'stream' else 'rows'}_gfx950",
+                grid=(SPLIT_GRID, 1, 1), block=(512, 1, 1), lds=split_lds_bytes(), dyn=0,
+                args=["x_q", "x_scale", "w13", "w13_scale", *routing, "h_q", "h_scale",
+                      u(cfg.T), u(cfg.I), u(cfg.Etot), u(cfg.cap_blocks)],
+                reads=["x_q", "x_scale", "w13", "w13_scale", *routing], writes=["h_q", "h_scale"],
+                refs=["kernels/gfx950/templates/moe/decode/gate_up_mfma.inc:12-161",
+                      "kernels/gfx950/templates/moe/decode/silu_quant.inc:16-236"])
 
 
 FRONTS = ("exact", "screen")
@@ -643,6 +678,8 @@ def operations(cfg: MoEConfig, path: str = "auto", front: str = "auto") -> list[
             gate_up,
             _tile_down(cfg),
         ]
+    if split_gate_up(cfg, path):
+        ops[-2] = _split_gate_up(cfg, path)
     combine_sym, combine_cols = ("netra_moe_combine_gfx950", 1024) if path == "stream" else \
         ("netra_moe_combine_bf16_gfx950", 2048)
     ops.append(
