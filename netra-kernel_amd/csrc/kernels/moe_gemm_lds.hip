@@ -93,6 +93,16 @@ __device__ __forceinline__ void copy16(uint32_t m0, u32x4 r, uint32_t voff, uint
                : "memory");
 }
 
+// copy16 with a non-temporal load, for weights a launch reads about once.
+__device__ __forceinline__ void copy16_once(uint32_t m0, u32x4 r, uint32_t voff, uint32_t soff) {
+  uint32_t saved;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds\n\t"
+               "s_mov_b32 m0, %0"
+               : "=&s"(saved)
+               : "s"(m0), "v"(voff), "s"(r), "s"(soff)
+               : "memory");
+}
+
 // 4 bytes per lane, global (rsrc + voff + soff) -> LDS (m0 + 4 * lane); as copy16.
 __device__ __forceinline__ void copy4(uint32_t m0, u32x4 r, uint32_t voff, uint32_t soff) {
   uint32_t saved;
@@ -154,7 +164,16 @@ __device__ __forceinline__ bool xcd_item(uint32_t i, uint32_t n, uint32_t& item)
 // rows I..2I-1 as plain row tiles) instead of the gate/up-interleaved
 // tile16x128 layout; the copies move the same 2 KiB blocks, only the up tile's
 // place and the operand reads out of LDS differ.
-template <uint32_t KB, bool kAiter = false>  // H / 128
+// kChoose: an item whose expert has no other block pair copies W13 with
+// non-temporal loads (no other item reads that slice, and its lines leave the
+// activations in the L2); with more pairs the copies are ordinary, and the
+// pairs' items find each other's lines there. gate/up us at H 2048, I 512, E
+// 256, K 8, all ordinary / all non-temporal / chosen: T = 512 113.1 / 107.0 /
+// 106.0, 1000 115.9 / 110.9 / 108.9, 2048 121.7 / 119.6 / 119.1, 4096 145.4 /
+// 149.8 / 145.4; Zipf-skewed 512 46.2 / 43.3 / 41.1, 1000 60.8 / 61.0 / 56.9,
+// 4096 140.1 / 147.7 / 137.2. (H 1024, whose tens of MB of weights the caches
+// hold: 39.4 / 44.2 at T = 2000, E 24, so only H 2048 chooses.)
+template <uint32_t KB, bool kAiter = false, bool kChoose = false>  // H / 128
 __device__ __forceinline__ void gate_up_lds(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13,
     const float* __restrict__ w13s, const int32_t* __restrict__ sorted_ids,
@@ -250,12 +269,16 @@ __device__ __forceinline__ void gate_up_lds(
   const uint32_t bvoff = lane * 16u;
   const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_offset(&s_stage[0][0]));
   // copy q = 0..6 of step kb (A halves, gate halves, up halves, tail share) into its stage
-  auto issue_part = [&](uint32_t kb, uint32_t q) __attribute__((always_inline)) {
+  auto issue_part = [&](uint32_t kb, uint32_t q, auto oncec) __attribute__((always_inline)) {
+    auto copy_w = [&](uint32_t m0, u32x4 r, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
+      if constexpr (decltype(oncec)::value) copy16_once(m0, r, voff, soff);
+      else copy16(m0, r, voff, soff);
+    };
     const uint32_t st = lds0 + (kb % kStages) * kStageBytes;
     const uint32_t half = (q & 1u) * 1024u;
     if (q < 2u) copy16(st + wave * 2048u + half, ra, avoff[q], kb * 128u);
-    else if (q < 4u) copy16(st + kABytes + wave * 2048u + half, rg, bvoff + half, kb * 2048u);
-    else if (q < 6u) copy16(st + kABytes + (8u + wave) * 2048u + half, rg, bvoff + half, (up_tiles * KB + kb) * 2048u);
+    else if (q < 4u) copy_w(st + kABytes + wave * 2048u + half, rg, bvoff + half, kb * 2048u);
+    else if (q < 6u) copy_w(st + kABytes + (8u + wave) * 2048u + half, rg, bvoff + half, (up_tiles * KB + kb) * 2048u);
     else copy16(st + kTailTile * 2048u + (wave & 1u) * 1024u, ra, tvoff, kb * 128u);
   };
   // The scales travel with the first step's copies (so no further round trip
@@ -291,16 +314,16 @@ __device__ __forceinline__ void gate_up_lds(
     for (uint32_t c = 0; c < 4; ++c) acc[i][c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   // the tail tile against this wave's gate and up tiles 2 n + m (16 h columns)
   v4f acc_t[2] = {v4f{0.0f, 0.0f, 0.0f, 0.0f}, v4f{0.0f, 0.0f, 0.0f, 0.0f}};
-  auto kloop = [&](auto ntc, auto tailc) __attribute__((always_inline)) {
+  auto kloop = [&](auto ntc, auto tailc, auto oncec) __attribute__((always_inline)) {
     constexpr uint32_t NT = decltype(ntc)::value;
     constexpr bool kTail = decltype(tailc)::value;
     // copies per step: the tail share only in the tail variant
     constexpr uint32_t kCopies = kTail ? kCopiesPerWave : kCopiesPerWave - 1u;
 #pragma unroll
-    for (uint32_t q = 0; q < kCopies; ++q) issue_part(0, q);
+    for (uint32_t q = 0; q < kCopies; ++q) issue_part(0, q, oncec);
     if (KB > 1)
 #pragma unroll
-      for (uint32_t q = 0; q < kCopies; ++q) issue_part(1, q);
+      for (uint32_t q = 0; q < kCopies; ++q) issue_part(1, q, oncec);
 #pragma unroll
     for (uint32_t kb = 0; kb < KB; ++kb) {
       if (kb + 1u < KB) wait_copies<kCopies>(); else wait_copies<0>();
@@ -312,7 +335,7 @@ __device__ __forceinline__ void gate_up_lds(
       auto some_copies = [&](uint32_t count) __attribute__((always_inline)) {
 #pragma unroll
         for (uint32_t u = 0; u < kCopies; ++u)
-          if (u < count && q < kCopies && kb + 2u < KB) { issue_part(kb + 2u, q); ++q; }
+          if (u < count && q < kCopies && kb + 2u < KB) { issue_part(kb + 2u, q, oncec); ++q; }
       };
       if (kb == 0) wsv = s_wsv[lane];  // the scale copy landed with step 0's copies
       if (NT > 0) {
@@ -358,16 +381,24 @@ __device__ __forceinline__ void gate_up_lds(
     }
   };
   using no_tail = std::false_type;
-  if (absorb) {
-    kloop(std::integral_constant<uint32_t, 4>{}, std::true_type{});
-  } else {
+  auto by_tiles = [&](auto oncec) __attribute__((always_inline)) {
     switch (ntiles) {
-      case 0: kloop(std::integral_constant<uint32_t, 0>{}, no_tail{}); break;
-      case 1: kloop(std::integral_constant<uint32_t, 1>{}, no_tail{}); break;
-      case 2: kloop(std::integral_constant<uint32_t, 2>{}, no_tail{}); break;
-      case 3: kloop(std::integral_constant<uint32_t, 3>{}, no_tail{}); break;
-      default: kloop(std::integral_constant<uint32_t, 4>{}, no_tail{}); break;
+      case 0: kloop(std::integral_constant<uint32_t, 0>{}, no_tail{}, oncec); break;
+      case 1: kloop(std::integral_constant<uint32_t, 1>{}, no_tail{}, oncec); break;
+      case 2: kloop(std::integral_constant<uint32_t, 2>{}, no_tail{}, oncec); break;
+      case 3: kloop(std::integral_constant<uint32_t, 3>{}, no_tail{}, oncec); break;
+      default: kloop(std::integral_constant<uint32_t, 4>{}, no_tail{}, oncec); break;
     }
+  };
+  // kChoose: whether this item alone reads its W13 slice (the expert has no
+  // other pair; an absorbed tail ends it)
+  const bool alone = kChoose && ep != e && (!two || e3 != e);
+  if (absorb) {
+    kloop(std::integral_constant<uint32_t, 4>{}, std::true_type{}, std::integral_constant<bool, kChoose>{});
+  } else if (alone) {  // uniform
+    by_tiles(std::integral_constant<bool, kChoose>{});
+  } else {
+    by_tiles(std::false_type{});
   }
   // Epilogue: h = bf16(silu(g) * u); amax per row over the 128-column group
   // (in stage KB % 3, which no wave reads after the K loop); FP8 bytes
@@ -455,7 +486,7 @@ __device__ __forceinline__ void gate_up_lds(
 }
 }  // namespace nklds
 
-#define NK_GATE_UP_LDS(HV)                                                                         \
+#define NK_GATE_UP_LDS(HV, CHOOSE)                                                                 \
   NK_KERNEL __launch_bounds__(512) void netra_moe_gate_up_lds_h##HV##_gfx950(                      \
       const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13, \
       const float* __restrict__ w13s, const int32_t* __restrict__ sorted_ids,                      \
@@ -463,12 +494,12 @@ __device__ __forceinline__ void gate_up_lds(
       const int32_t* __restrict__ pair_map, uint8_t* __restrict__ hq, float* __restrict__ hs,      \
       uint32_t T, uint32_t H, uint32_t I, uint32_t Ktot, uint32_t Etot) {                          \
     (void)H;                                                                                       \
-    nklds::gate_up_lds<HV / 128>(xq, xs, w13, w13s, sorted_ids, sorted_expert, num_valid,          \
-                                 pair_map, hq, hs, T, I, Ktot, Etot);                              \
+    nklds::gate_up_lds<HV / 128, false, CHOOSE>(xq, xs, w13, w13s, sorted_ids, sorted_expert,      \
+                                                num_valid, pair_map, hq, hs, T, I, Ktot, Etot);    \
   }
-NK_GATE_UP_LDS(512)
-NK_GATE_UP_LDS(1024)
-NK_GATE_UP_LDS(2048)
+NK_GATE_UP_LDS(512, false)
+NK_GATE_UP_LDS(1024, false)
+NK_GATE_UP_LDS(2048, true)
 
 // W13 in the reference's AITER layout (the M768 prefill bridge): same ABI.
 #define NK_GATE_UP_LDS_AITER(HV)                                                                   \

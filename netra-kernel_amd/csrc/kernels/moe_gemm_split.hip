@@ -46,7 +46,6 @@ using nkstream::lds_barrier;
 
 constexpr uint32_t kMaxE = 513;             // experts, the shared one included
 constexpr uint32_t kPer = (kMaxE + 63) / 64;  // experts per lane of the scan
-constexpr int kNt = 2;                      // buffer aux bit: non-temporal
 
 struct Table {
   uint32_t n[kMaxE];        // rows of each expert
@@ -132,15 +131,6 @@ __device__ __forceinline__ void share(uint32_t total, uint32_t& lo, uint32_t& hi
   if (gridDim.x % 8u == 0u) w = (w & 7u) * (gridDim.x / 8u) + (w >> 3);
   lo = (uint32_t)((uint64_t)w * total / gridDim.x);
   hi = (uint32_t)((uint64_t)(w + 1u) * total / gridDim.x);
-}
-
-__device__ __forceinline__ v8i load_operand_nt(__amdgpu_buffer_rsrc_t r, uint32_t tile_offset, uint32_t lane) {
-  const nk::u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(lane * 16u), (int)tile_offset, kNt);
-  const nk::u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(lane * 16u + 1024u), (int)tile_offset, kNt);
-  v8i v;
-  v[0] = (int)lo.x; v[1] = (int)lo.y; v[2] = (int)lo.z; v[3] = (int)lo.w;
-  v[4] = (int)hi.x; v[5] = (int)hi.y; v[6] = (int)hi.z; v[7] = (int)hi.w;
-  return v;
 }
 
 __device__ __forceinline__ float lane_f32(float v, uint32_t l) {
@@ -230,13 +220,13 @@ __device__ __forceinline__ void gate_up_split(
       const uint32_t c = (2u * ip + j) * CA + ca;
       b.ws = wse[(live ? c >> 3 : 0u) * KB];  // (ahead of the tiles it scales)
 #pragma unroll
-      for (uint32_t i = 0; i < KBW; ++i) b.g[i] = load_operand_nt(r, (2u * c * KB + kb0 + i) * 2048u, lane);
+      for (uint32_t i = 0; i < KBW; ++i) b.g[i] = nk::load_tile_operand<false, true>(r, (2u * c * KB + kb0 + i) * 2048u, lane);
     };
     auto issue_u = [&](GuBuf<KBW>& b, uint32_t ip, uint32_t j, bool live) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t r = nk::buffer_rsrc(we, live ? 2u * I * H : 0u);
       const uint32_t c = (2u * ip + j) * CA + ca;
 #pragma unroll
-      for (uint32_t i = 0; i < KBW; ++i) b.u[i] = load_operand_nt(r, ((2u * c + 1u) * KB + kb0 + i) * 2048u, lane);
+      for (uint32_t i = 0; i < KBW; ++i) b.u[i] = nk::load_tile_operand<false, true>(r, ((2u * c + 1u) * KB + kb0 + i) * 2048u, lane);
     };
     // the chunk's rows: lane l holds row l & 15 of every tile
     v8i a[R][KBW];

@@ -400,7 +400,14 @@ __device__ __forceinline__ uint16_t f16_bits(float x) {
   return __builtin_bit_cast(uint16_t, h);
 }
 
-template <uint32_t KB, bool kAiter = false, bool kSplitF16 = false>  // I / 128
+// kChoose: an expert with one block reads its W2 with non-temporal loads (no other item
+// shares those lines, and the L2 keeps the activations); an expert with more
+// keeps ordinary loads, whose lines its other blocks' items find in the L2.
+// down us at H 2048, I 512, E 256, K 8, all ordinary / all non-temporal /
+// chosen: T = 257 62.4 / 53.6 / 54.0, 512 64.8 / 57.0 / 57.4, 1000 72.1 / 62.2 /
+// 62.8, 2048 83.8 / 84.3 / 78.9, 4096 107 / 141 / 107; Zipf-skewed 512 28.5 /
+// 29.6 / 26.9, 1000 39.3 / 39.5 / 35.4.
+template <uint32_t KB, bool kAiter = false, bool kSplitF16 = false, bool kChoose = false>  // I / 128
 __device__ __forceinline__ void down_rows(
     const uint8_t* __restrict__ hq, const float* __restrict__ hs, const uint8_t* __restrict__ w2,
     const float* __restrict__ w2s, const int32_t* __restrict__ sorted_ids,
@@ -429,24 +436,32 @@ __device__ __forceinline__ void down_rows(
   uint32_t item;
   if (!xcd_item(blockIdx.x, ((uint32_t)num_valid[0] / kRows) * NCH, item)) return;
   const uint32_t b = item / NCH, nb0 = (item - b * NCH) * NBC;
+  const uint32_t nblocks = (uint32_t)num_valid[0] / kRows;
   const int32_t e = sorted_expert[b];
+  const bool alone = kChoose && (b == 0u || sorted_expert[b - 1u] != e) && (b + 1u >= nblocks || sorted_expert[b + 1u] != e);
   if (e < 0 || (uint32_t)e >= Etot) return;
   if (tid < kRows) {
     const int32_t id = sorted_ids[b * kRows + tid];
     const uint32_t t = (uint32_t)id & 0xffffffu, slot = (uint32_t)id >> 24;
     s_route[tid] = (t < T && slot < Ktot) ? (int32_t)(t * Ktot + slot) : -1;
   }
+  // the item from its weights on, kOnce: W2 non-temporal
+  auto item_body = [&](auto oncec) __attribute__((always_inline)) {
+  constexpr bool kOnce = decltype(oncec)::value;
   // The expert's W2 in tile16x128 (row tile rt's K blocks contiguous); wave
   // w's tile of group nb is row tile 8 nb + w. Its weight scales come one per
   // lane (lane kb holds w_s(nb, kb)) by a vector load: a scalar load would
   // share the LDS counter and make the next LDS wait a full drain.
   const __amdgpu_buffer_rsrc_t wt = nk::buffer_rsrc(w2 + (size_t)e * H * I, H * I);
-  const float* wse = w2s + (size_t)e * NB * KB;
+  const __amdgpu_buffer_rsrc_t wsr = nk::buffer_rsrc(w2s + (size_t)e * NB * KB, NB * KB * 4u);
+  auto load_ws = [&](uint32_t nb) __attribute__((always_inline)) {  // lane kb: group nb's K block kb
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wsr, (int)((lane & (KB - 1u)) * 4u), (int)(nb * KB * 4u), 0));
+  };
   v8i bq[KB];
 #pragma unroll
   for (uint32_t kb = 0; kb < KB; ++kb)
-    bq[kb] = nk::load_tile_operand<kAiter>(wt, ((nb0 * 8u + wave) * KB + kb) * 2048u, lane);
-  float wsv = wse[nb0 * KB + (lane & (KB - 1u))];
+    bq[kb] = nk::load_tile_operand<kAiter, kOnce>(wt, ((nb0 * 8u + wave) * KB + kb) * 2048u, lane);
+  float wsv = load_ws(nb0);
   // the block's A rows (64 x I bytes, contiguous) and scales; thread slot s
   // of the operand layout fetches the 16 bytes that belong there
   constexpr uint32_t kA16 = kRows * I / 16u / kThreads;  // uint4 per thread
@@ -530,7 +545,7 @@ __device__ __forceinline__ void down_rows(
     constexpr bool kRefill = decltype(refc)::value;
     {
       const uint32_t nb = nb0 + q, nbn = nb0 + (kRefill && q + 1u < NBC ? q + 1u : q);
-      const float wsn = kRefill ? wse[nbn * KB + (lane & (KB - 1u))] : 0.0f;
+      const float wsn = kRefill ? load_ws(nbn) : 0.0f;
       v4f acc[NT];
 #pragma unroll
       for (uint32_t rt = 0; rt < NT; ++rt) acc[rt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -542,7 +557,7 @@ __device__ __forceinline__ void down_rows(
         for (uint32_t rt = 0; rt < NT; ++rt)
           d[rt] = nk::mfma_e4m3_16x16x128(bq[kb], nk::load_tile_operand(&s_a[(rt * KB + kb) * 2048u], lane));
         if constexpr (kRefill)  // the next group's tile
-          bq[kb] = nk::load_tile_operand<kAiter>(wt, ((nbn * 8u + wave) * KB + kb) * 2048u, lane);
+          bq[kb] = nk::load_tile_operand<kAiter, kOnce>(wt, ((nbn * 8u + wave) * KB + kb) * 2048u, lane);
 #pragma unroll
         for (uint32_t rt = 0; rt < NT; ++rt) {
           const float sc = ws * s_hs[kb * kRows + rt * 16u + (lane & 15u)];  // this lane's route row
@@ -586,6 +601,9 @@ __device__ __forceinline__ void down_rows(
     case 3: run(std::integral_constant<uint32_t, 3>{}); break;
     default: run(std::integral_constant<uint32_t, 4>{}); break;
   }
+  };
+  if (alone) item_body(std::integral_constant<bool, kChoose>{});  // uniform
+  else item_body(std::false_type{});
 }
 
 }  // namespace nktile
@@ -626,7 +644,7 @@ NK_DOWN_TILE(512)
 NK_DOWN_TILE(1024)
 
 #define NK_DOWN_ROWS(IV)                                                                           \
-  NK_KERNEL __launch_bounds__(512)                                                                \
+  NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))                        \
   void netra_moe_down_rows_i##IV##_gfx950(                                                        \
       const uint8_t* __restrict__ hq, const float* __restrict__ hs, const uint8_t* __restrict__ w2, \
       const float* __restrict__ w2s, const int32_t* __restrict__ sorted_ids,                       \
@@ -634,8 +652,8 @@ NK_DOWN_TILE(1024)
       uint16_t* __restrict__ partial, uint32_t T, uint32_t H, uint32_t I, uint32_t Ktot,           \
       uint32_t Etot, uint32_t NBC) {                                                               \
     (void)I;                                                                                       \
-    nktile::down_rows<IV / 128>(hq, hs, w2, w2s, sorted_ids, sorted_expert, num_valid, partial, T, \
-                                H, Ktot, Etot, NBC);                                               \
+    nktile::down_rows<IV / 128, false, false, true>(hq, hs, w2, w2s, sorted_ids, sorted_expert,    \
+                                                    num_valid, partial, T, H, Ktot, Etot, NBC);    \
   }
 NK_DOWN_ROWS(256)
 NK_DOWN_ROWS(512)

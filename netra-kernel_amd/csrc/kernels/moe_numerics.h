@@ -195,11 +195,13 @@ __device__ __forceinline__ v8i load_block_operand(const uint8_t* tile, uint32_t 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
-template <bool kAiter = false>
+// kOnce: non-temporal loads.
+template <bool kAiter = false, bool kOnce = false>
 __device__ __forceinline__ v8i load_tile_operand(__amdgpu_buffer_rsrc_t r, uint32_t tile_offset,
                                                  uint32_t lane) {
-  const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(r, (int)operand_lo<kAiter>(lane), (int)tile_offset, 0);
-  const u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(r, (int)operand_hi<kAiter>(lane), (int)tile_offset, 0);
+  constexpr int kAux = kOnce ? 2 : 0;  // the nt bit
+  const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(r, (int)operand_lo<kAiter>(lane), (int)tile_offset, kAux);
+  const u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(r, (int)operand_hi<kAiter>(lane), (int)tile_offset, kAux);
   v8i v;
   v[0] = (int)lo.x; v[1] = (int)lo.y; v[2] = (int)lo.z; v[3] = (int)lo.w;
   v[4] = (int)hi.x; v[5] = (int)hi.y; v[6] = (int)hi.z; v[7] = (int)hi.w;
