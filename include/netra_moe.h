@@ -63,6 +63,9 @@
 //   netra_moe_ffn_down_h2048_i512_single_gfx950(the same arguments)   T = 1,
 //       grid H/16, block 512: a workgroup owns 16 output columns across all
 //       routes and writes out itself (partial for inspection; counters unused)
+//   netra_moe_ffn_gate_up_h<H>_i<I>_wide_p<P>_gfx950(the wide gate/up's arguments)   P
+//       128-column blocks of h per workgroup instead of min(4, I / 128), for calls
+//       with few tiles
 //   netra_moe_ffn_gate_up_down_h<H>_i<I>[_ksplit]_gfx950(the gate/up arguments, with w2,
 //       w2s and partial f32[T*Ktot,H] after hs)   (H, I) in {(512,256), (2048,512)}
 //       (_ksplit: (2048,512) only), grid 256, block 512: the wide gate/up (_ksplit: K
@@ -86,6 +89,10 @@
 //       w2s f32[Etot,H/128,I/128], sorted_ids, sorted_expert, tile_map, num_valid,
 //       partial f32[T*Ktot,H]; T, H, I, Ktot, Etot)   grid 2048, block 256
 //       (DC K blocks per step, 1 or 2)
+//   few rows per expert (T * K <= 13 E), H = 2048, I = 512:
+//   netra_moe_gate_up_split_h2048_<tiles|rows>_gfx950(xq, xs, w13, w13s, sorted_ids, counts,
+//       hq, hs; T, I, Etot, CAP)   grid 256, block 512, static LDS 149 KiB, T*H < 2^31, CAP <
+//       65536; hq / hs as gate_up_stream's (tiles) or gate_up_lds' (rows)
 //   prefill ("tile") GEMMs, H in {512,1024,2048,4096}, I in {256,512,1024}:
 //   netra_moe_gate_up_tile_h<H>_gfx950(xq, xs, w13, w13s, sorted_ids, sorted_expert,
 //       num_valid, hq e4m3[CAP*64,I], hs f32[CAP*64,I/128]; T, H, I, Ktot, Etot)

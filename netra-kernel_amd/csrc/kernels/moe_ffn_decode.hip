@@ -24,6 +24,7 @@
 //     requantised h in its LDS (fp32 partials to the combine kernel); _ksplit
 //     splits gate/up's K over the waves. Chosen when a call has enough tiles
 //     to keep the chip streaming.
+//   netra_moe_ffn_gate_up_h<H>_i<I>_wide_p<P>_gfx950(as wide)   fewer columns per workgroup
 //   block 512 (8 waves), any grid
 // Weights are read with non-temporal loads: every tile is read by one
 // workgroup per launch (the tiles of an expert with more than 16 routes by
@@ -1274,6 +1275,33 @@ NK_FFN_PAIR(2048, 512, wide, 1, 1, 2, 2, 4, 2, 4, 1)
 NK_FFN_PAIR(2048, 512, narrow, 8, 4, 1, 4, 1, 1, 4, 1)
 NK_FFN_PAIR(4096, 256, wide, 1, 1, 2, 2, 2, 2, 4, 1)
 NK_FFN_PAIR(4096, 256, narrow, 8, 2, 2, 2, 1, 1, 4, 1)
+
+// Symbols netra_moe_ffn_gate_up_h<H>_i<I>_wide_p<P>_gfx950: the wide gate/up with
+// fewer column items per wave (P 128-column blocks of h per workgroup instead of
+// the whole tile), for calls whose tiles are too few to fill the chip: one
+// workgroup's weight stream is bound by its own latency (42 GB/s at two steps of
+// 64 KiB in flight), not by the HBM. H 1024, I 1024, 27 tiles: 26.8 -> 14.1 us;
+// H 4096, I 256, 37 tiles: 47.1 -> 29.2 us; H 2048, I 512, 108 tiles: 49.7 -> 43.1.
+#define NK_FFN_GATE_UP_SPREAD(HV, IV, PG)                                                           \
+  NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))                         \
+  void netra_moe_ffn_gate_up_h##HV##_i##IV##_wide_p##PG##_gfx950(                                  \
+      const uint16_t* __restrict__ logits, const float* __restrict__ bias,                         \
+      int32_t* __restrict__ topk_ids, float* __restrict__ topk_weights, const uint8_t* __restrict__ xq, \
+      const float* __restrict__ xs, const uint8_t* __restrict__ w13, const float* __restrict__ w13s, \
+      int32_t* __restrict__ sorted_ids, int32_t* __restrict__ sorted_expert,                       \
+      int32_t* __restrict__ tile_map, int32_t* __restrict__ pair_map, int32_t* __restrict__ num_valid, \
+      int32_t* __restrict__ counts, uint16_t* __restrict__ hrows, uint8_t* __restrict__ hq,        \
+      float* __restrict__ hs, uint32_t T, uint32_t E, uint32_t K, uint32_t S, uint32_t cap_blocks) { \
+    nkffn::ffn_gate_up<HV / 128, IV / 128, 1, 2, PG>(logits, bias, topk_ids, topk_weights, xq, xs, w13, \
+                                                     w13s, sorted_ids, sorted_expert, tile_map,    \
+                                                     pair_map, num_valid, counts, hrows, hq, hs, T, \
+                                                     E, K, S, cap_blocks);                         \
+  }
+NK_FFN_GATE_UP_SPREAD(1024, 1024, 1)
+NK_FFN_GATE_UP_SPREAD(1024, 1024, 2)
+NK_FFN_GATE_UP_SPREAD(2048, 512, 1)
+NK_FFN_GATE_UP_SPREAD(2048, 512, 2)
+NK_FFN_GATE_UP_SPREAD(4096, 256, 1)
 
 // Symbols netra_moe_ffn_gate_up_down_h<H>_i<I>[_ksplit]_gfx950: the wide gate/up
 // with each tile's down in the same workgroup (the tile's h requantised into

@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import hashlib
 import json
+import math
 import shutil
 from dataclasses import dataclass
 from pathlib import Path
@@ -489,13 +490,35 @@ def down_variant(cfg: MoEConfig) -> str:
     return "rows" if v == "narrow" and cfg.T >= NARROW_ROWS_DOWN_T else v
 
 
+# (H, I) -> smaller P of the wide gate/up (netra_moe_ffn_gate_up_h<H>_i<I>_wide_p<P>)
+FFN_SPREAD_P = {(1024, 1024): (1, 2), (2048, 512): (1, 2), (4096, 256): (1,)}
+
+
+def ffn_wide_p(cfg: MoEConfig) -> int:
+    """Column items per wave of the wide gate/up: a workgroup streams P
+    128-column blocks of a tile, so the full P leaves most CUs idle when a call
+    has few tiles, and a smaller one costs rounds when it has many. A smaller P
+    is taken where it at least halves rounds x P (the expected items with 6%
+    for the spread of the routing, over 256 workgroups), the larger of equals.
+    Gate/up µs, full / chosen: H 1024, I 1024, E 24, K 3, T = 20 26.0 / 13.1, 40
+    26.8 / 14.1, 64 27.5 / 14.9; H 4096, I 256, E 32, K 4, T = 20 44.9 / 27.7, 64
+    47.1 / 29.2; H 2048, I 512, E 256, K 8, T = 17 (108 tiles) 49.7 / 43.1, 19
+    (118) 54.1 / 48.3, and at 21 (127, where it would cost a second round of P
+    = 2 or a third of 1) 54.6 / 63.3 and 56.3."""
+    full = FFN_WIDE_P[(cfg.H, cfg.I)]
+    tiles, blocks = expected_tiles(cfg), cfg.I // 128
+    cost = lambda p: math.ceil(1.06 * tiles * (blocks // p) / FFN_GRID[("gate_up", "wide")]) * p  # noqa: E731
+    best = min(FFN_SPREAD_P.get((cfg.H, cfg.I), ()), key=lambda p: (cost(p), -p), default=full)
+    return best if 2 * cost(best) <= cost(full) else full
+
+
 def ffn_lds_bytes(cfg: MoEConfig) -> tuple[int, int]:
     """Static LDS of netra_moe_ffn_{gate_up,down}_h<H>_i<I>_<v> (their
     __shared__ arrays, rounded up)."""
     kb, kbi = cfg.H // 128, cfg.I // 128
     narrow = ffn_variant(cfg) == "narrow"
     red = 8 * 8 * 64 * 4 if narrow else 0
-    gu = max(kb * 2048, red, 1024 * 4 + 513 * 4) + 64 * kb + (8 if narrow else 16 * (128 * FFN_WIDE_P[(cfg.H, cfg.I)] + 8)) * 2
+    gu = max(kb * 2048, red, 1024 * 4 + 513 * 4) + 64 * kb + (8 if narrow else 16 * (128 * ffn_wide_p(cfg) + 8)) * 2
     gu += 64 * 16 * 4 + 512 * 8 + 2 * 513 * 4 + 48 * 4
     if down_variant(cfg) == "merged" and expected_tiles(cfg) >= MERGED_KSPLIT_MIN_TILES.get((cfg.H, cfg.I), float("inf")):
         gu += 2 * 8 * 8 * 64 * 4  # the K split's sums, two steps
@@ -535,9 +558,10 @@ def _fused_decode(cfg: MoEConfig) -> list[dict]:
     narrow = v == "narrow"
     route = _router_logits_op(cfg) if narrow else _route_op(cfg)
     topk = ["topk_ids", "topk_weights"]
+    spread = "" if narrow or ffn_wide_p(cfg) == FFN_WIDE_P[(H, I)] else f"_p{ffn_wide_p(cfg)}"
     ops = [
         route,
-        dict(name="moe.gate_up", symbol=f"netra_moe_ffn_gate_up_h{H}_i{I}_{v}_gfx950",
+        dict(name="moe.gate_up", symbol=f"netra_moe_ffn_gate_up_h{H}_i{I}_{v}{spread}_gfx950",
              grid=(ffn_grid(cfg, "gate_up"), 1, 1), block=(512, 1, 1), lds=lds_gu, dyn=0,
              args=["logits", "router_bias", *topk, "x_q", "x_scale", "w13", "w13_scale", *sort_out,
                    "h_rows", "h_q", "h_scale", u(T), u(cfg.E), u(cfg.K), u(cfg.S), u(cfg.cap_blocks)],
