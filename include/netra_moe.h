@@ -102,12 +102,12 @@
 //       grid 8*ceil(CAP*I/128/8), block 512, static LDS <= 155 KiB, T*H < 2^31;
 //       one item per (block pair, 128 h columns), assigned XCD-major
 //   netra_moe_down_rows_i<I>_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert, num_valid,
-//       partial bf16[T*Ktot,H]; T, H, I, Ktot, Etot, NBC)   I in {256,512},
+//       partial bf16[T*Ktot,H]; T, H, I, Ktot, Etot, NBC)   I in {256,512,1024},
 //       grid 8*ceil(CAP*(H/128/NBC)/8), block 512, T*Ktot*H*2 < 2^31; one item per
 //       (64-row block, NBC consecutive 128-column groups), NBC divides H/128
 //   netra_moe_down_tile_i<I>_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert, num_valid,
 //       partial bf16[T*Ktot,H]; T, H, I, Ktot, Etot)   grid 8*ceil(CAP*H/128/8), block 256;
-//       used for I = 1024
+//       used for I = 1024 with few blocks, and where partial has 2^31 bytes or more
 //   netra_moe_combine_gfx950(partial f32, weights, out bf16[T,H]; T, H, Ktot)
 //       grid (ceil(H/1024), T), block 256
 //   netra_moe_combine_bf16_gfx950(partial bf16, weights, out; T, H, Ktot)

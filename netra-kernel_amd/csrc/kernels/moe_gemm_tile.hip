@@ -643,8 +643,8 @@ NK_DOWN_TILE(256)
 NK_DOWN_TILE(512)
 NK_DOWN_TILE(1024)
 
-#define NK_DOWN_ROWS(IV)                                                                           \
-  NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))                        \
+#define NK_DOWN_ROWS(IV, WPE, CHOOSE)                                                               \
+  NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE)))                      \
   void netra_moe_down_rows_i##IV##_gfx950(                                                        \
       const uint8_t* __restrict__ hq, const float* __restrict__ hs, const uint8_t* __restrict__ w2, \
       const float* __restrict__ w2s, const int32_t* __restrict__ sorted_ids,                       \
@@ -652,11 +652,12 @@ NK_DOWN_TILE(1024)
       uint16_t* __restrict__ partial, uint32_t T, uint32_t H, uint32_t I, uint32_t Ktot,           \
       uint32_t Etot, uint32_t NBC) {                                                               \
     (void)I;                                                                                       \
-    nktile::down_rows<IV / 128, false, false, true>(hq, hs, w2, w2s, sorted_ids, sorted_expert,    \
+    nktile::down_rows<IV / 128, false, false, CHOOSE>(hq, hs, w2, w2s, sorted_ids, sorted_expert,    \
                                                     num_valid, partial, T, H, Ktot, Etot, NBC);    \
   }
-NK_DOWN_ROWS(256)
-NK_DOWN_ROWS(512)
+NK_DOWN_ROWS(256, 4, true)
+NK_DOWN_ROWS(512, 4, true)
+NK_DOWN_ROWS(1024, 2, false)  // 100 KiB of LDS: one workgroup per CU
 
 // The M768 prefill bridge's producer format: W2 in the AITER layout, fp16
 // split-K2 route partials (half 1 starts half_rows rows after half 0).

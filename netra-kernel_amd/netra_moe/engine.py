@@ -62,8 +62,13 @@ STREAM_H = (512, 1024, 2048, 4096)   # netra_moe_gate_up_stream_h<H>_c<CH>_gfx95
 STREAM_I = (256, 512, 1024, 2048)    # netra_moe_down_stream_i<I>_c<DC>_gfx950
 TILE_H = (512, 1024, 2048, 4096)     # netra_moe_gate_up_tile_h<H>_gfx950
 TILE_I = (256, 512, 1024)            # netra_moe_down_tile_i<I>_gfx950
-ROWS_I = (256, 512)                  # netra_moe_down_rows_i<I>_gfx950 (block rows x runs of column groups)
-DOWN_ROWS_ITEMS = 1024               # down_rows: fewer column groups per item until about this many items
+ROWS_I = (256, 512, 1024)            # netra_moe_down_rows_i<I>_gfx950 (block rows x runs of column groups)
+# down_rows: fewer column groups per item until about this many items (I 1024:
+# one workgroup per CU fits and an item stages 64 KiB of rows; down µs at H
+# 1024, E 24, K 3 with 1024 / 256 / 128: T = 600 18.4 / 18.6 / 14.5, 1000 26.5 /
+# 23.3 / 20.0, 2000 41.7 / 32.5 / 30.1, 4000 56.0 / 57.3 / 54.9; the 128-column
+# down_tile 19.1, 26.0, 39.7, 65.9)
+DOWN_ROWS_ITEMS = {256: 1024, 512: 1024, 1024: 128}
 TILE_GU_WAVES = 4                    # waves of netra_moe_gate_up_tile_h<H>_gfx950 (its launch bound)
 SPLIT_HI = ((2048, 512),)            # netra_moe_gate_up_split_h<H>_{tiles|rows}_gfx950
 LDS_GU_H = (512, 1024, 2048)         # netra_moe_gate_up_lds_h<H>_gfx950: 128-row pairs, LDS operand ring
@@ -400,7 +405,7 @@ def down_rows_groups(cfg: MoEConfig) -> int:
     nb = cfg.H // 128
     blocks = (cfg.routes + 63) // 64 + min(cfg.Etot, cfg.routes) // 2  # expected non-empty blocks
     nbc = nb
-    while nbc > 1 and nbc % 2 == 0 and blocks * (nb // nbc) < DOWN_ROWS_ITEMS:
+    while nbc > 1 and nbc % 2 == 0 and blocks * (nb // nbc) < DOWN_ROWS_ITEMS[cfg.I]:
         nbc //= 2
     return nbc
 
@@ -616,8 +621,10 @@ def _tile_down(cfg: MoEConfig) -> dict:
     common = ["sorted_ids", "sorted_expert", "num_valid"]
     refs = ["kernels/gfx950/templates/moe/prefill/fused_splitk2/down_partial.inc",
             "kernels/gfx950/templates/moe/prefill/route_reduce_splitk2_f16.inc:6-117"]
-    if I in ROWS_I and cfg.routes * H * 2 < 1 << 31:
-        nbc = down_rows_groups(cfg)
+    nbc = down_rows_groups(cfg) if I in ROWS_I else 1
+    # (I 1024 at one group per item: the 64 KiB of rows are staged for one
+    # group, no faster than down_tile: T = 300, E 24, K 3 11.8 / 11.7 us)
+    if I in ROWS_I and (I < 1024 or nbc > 1) and cfg.routes * H * 2 < 1 << 31:
         return dict(name="moe.down", symbol=f"netra_moe_down_rows_i{I}_gfx950",
                     grid=(xcd_grid(cfg.cap_blocks * (H // 128 // nbc)), 1, 1), block=(512, 1, 1),
                     lds=64 * I + 2 * 64 * 272 + 64 * (I // 128) * 4 + 64 * 4, dyn=0,

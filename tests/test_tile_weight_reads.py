@@ -14,14 +14,15 @@ from netra_moe.config import MoEConfig
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
-@pytest.mark.parametrize("T", [64, 65, 128, 129, 144, 145, 257, 272])
-def test_experts_of_every_block_count(T):
+@pytest.mark.parametrize("T,H,I", [(t, 2048, 512) for t in (64, 65, 128, 129, 144, 145, 257, 272)]
+                         + [(t, 1024, 1024) for t in (300, 700, 2000)])  # I 1024: down_tile, down_rows of 2 and 4 groups
+def test_experts_of_every_block_count(T, H, I):
     import torch
 
     import oracle
     from moe_case import make_inputs, oracle_routing, run_gpu, sample_tokens
 
-    cfg = MoEConfig(f"reads_t{T}", T=T, H=2048, E=8, K=2, I=512, S=1, router_bias="hot", seed=1300 + T)
+    cfg = MoEConfig(f"reads_t{T}_h{H}", T=T, H=H, E=8, K=2, I=I, S=1, router_bias="hot", seed=1300 + T)
     print(f"\n[reads] {cfg}", flush=True)
     dev = torch.device("cuda", 0)
     x, gpu_w, host = make_inputs(cfg, dev)
