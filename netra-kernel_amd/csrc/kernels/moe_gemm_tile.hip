@@ -406,7 +406,10 @@ __device__ __forceinline__ uint16_t f16_bits(float x) {
 // down us at H 2048, I 512, E 256, K 8, all ordinary / all non-temporal /
 // chosen: T = 257 62.4 / 53.6 / 54.0, 512 64.8 / 57.0 / 57.4, 1000 72.1 / 62.2 /
 // 62.8, 2048 83.8 / 84.3 / 78.9, 4096 107 / 141 / 107; Zipf-skewed 512 28.5 /
-// 29.6 / 26.9, 1000 39.3 / 39.5 / 35.4.
+// 29.6 / 26.9, 1000 39.3 / 39.5 / 35.4. The choice is a uniform branch around
+// each pair of loads: two bodies, one for each kind, spilled a register at I
+// 512, and the scratch of every launch cost more than the branch (down at E
+// 16, K 4, T = 1040 23.5 -> 21.0 us; Zipf T = 512 28.0 -> 26.7).
 template <uint32_t KB, bool kAiter = false, bool kSplitF16 = false, bool kChoose = false>  // I / 128
 __device__ __forceinline__ void down_rows(
     const uint8_t* __restrict__ hq, const float* __restrict__ hs, const uint8_t* __restrict__ w2,
@@ -438,16 +441,20 @@ __device__ __forceinline__ void down_rows(
   const uint32_t b = item / NCH, nb0 = (item - b * NCH) * NBC;
   const uint32_t nblocks = (uint32_t)num_valid[0] / kRows;
   const int32_t e = sorted_expert[b];
-  const bool alone = kChoose && (b == 0u || sorted_expert[b - 1u] != e) && (b + 1u >= nblocks || sorted_expert[b + 1u] != e);
+  // kChoose: whether this is the expert's only block (the neighbours' experts
+  // are read unconditionally: one round trip)
+  bool alone = false;
+  if constexpr (kChoose) {
+    const bool before = b != 0u, after = b + 1u < nblocks;
+    const int32_t ep = sorted_expert[before ? b - 1u : b], en = sorted_expert[after ? b + 1u : b];
+    alone = !(before & (ep == e)) & !(after & (en == e));
+  }
   if (e < 0 || (uint32_t)e >= Etot) return;
   if (tid < kRows) {
     const int32_t id = sorted_ids[b * kRows + tid];
     const uint32_t t = (uint32_t)id & 0xffffffu, slot = (uint32_t)id >> 24;
     s_route[tid] = (t < T && slot < Ktot) ? (int32_t)(t * Ktot + slot) : -1;
   }
-  // the item from its weights on, kOnce: W2 non-temporal
-  auto item_body = [&](auto oncec) __attribute__((always_inline)) {
-  constexpr bool kOnce = decltype(oncec)::value;
   // The expert's W2 in tile16x128 (row tile rt's K blocks contiguous); wave
   // w's tile of group nb is row tile 8 nb + w. Its weight scales come one per
   // lane (lane kb holds w_s(nb, kb)) by a vector load: a scalar load would
@@ -457,10 +464,13 @@ __device__ __forceinline__ void down_rows(
   auto load_ws = [&](uint32_t nb) __attribute__((always_inline)) {  // lane kb: group nb's K block kb
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wsr, (int)((lane & (KB - 1u)) * 4u), (int)(nb * KB * 4u), 0));
   };
+  auto load_w = [&](uint32_t offset) __attribute__((always_inline)) {  // one weight tile
+    if (kChoose && alone) return nk::load_tile_operand<kAiter, true>(wt, offset, lane);  // uniform
+    return nk::load_tile_operand<kAiter>(wt, offset, lane);
+  };
   v8i bq[KB];
 #pragma unroll
-  for (uint32_t kb = 0; kb < KB; ++kb)
-    bq[kb] = nk::load_tile_operand<kAiter, kOnce>(wt, ((nb0 * 8u + wave) * KB + kb) * 2048u, lane);
+  for (uint32_t kb = 0; kb < KB; ++kb) bq[kb] = load_w(((nb0 * 8u + wave) * KB + kb) * 2048u);
   float wsv = load_ws(nb0);
   // the block's A rows (64 x I bytes, contiguous) and scales; thread slot s
   // of the operand layout fetches the 16 bytes that belong there
@@ -557,7 +567,7 @@ __device__ __forceinline__ void down_rows(
         for (uint32_t rt = 0; rt < NT; ++rt)
           d[rt] = nk::mfma_e4m3_16x16x128(bq[kb], nk::load_tile_operand(&s_a[(rt * KB + kb) * 2048u], lane));
         if constexpr (kRefill)  // the next group's tile
-          bq[kb] = nk::load_tile_operand<kAiter, kOnce>(wt, ((nbn * 8u + wave) * KB + kb) * 2048u, lane);
+          bq[kb] = load_w(((nbn * 8u + wave) * KB + kb) * 2048u);
 #pragma unroll
         for (uint32_t rt = 0; rt < NT; ++rt) {
           const float sc = ws * s_hs[kb * kRows + rt * 16u + (lane & 15u)];  // this lane's route row
@@ -601,9 +611,6 @@ __device__ __forceinline__ void down_rows(
     case 3: run(std::integral_constant<uint32_t, 3>{}); break;
     default: run(std::integral_constant<uint32_t, 4>{}); break;
   }
-  };
-  if (alone) item_body(std::integral_constant<bool, kChoose>{});  // uniform
-  else item_body(std::false_type{});
 }
 
 }  // namespace nktile
@@ -643,9 +650,10 @@ NK_DOWN_TILE(256)
 NK_DOWN_TILE(512)
 NK_DOWN_TILE(1024)
 
-#define NK_DOWN_ROWS(IV, WPE, CHOOSE)                                                               \
+// _once: kChoose (the engine's rule for it: engine.py, weights_once)
+#define NK_DOWN_ROWS(IV, NAME, WPE, CHOOSE)                                                         \
   NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE)))                      \
-  void netra_moe_down_rows_i##IV##_gfx950(                                                        \
+  void netra_moe_down_rows_##NAME##_gfx950(                                                       \
       const uint8_t* __restrict__ hq, const float* __restrict__ hs, const uint8_t* __restrict__ w2, \
       const float* __restrict__ w2s, const int32_t* __restrict__ sorted_ids,                       \
       const int32_t* __restrict__ sorted_expert, const int32_t* __restrict__ num_valid,            \
@@ -655,9 +663,11 @@ NK_DOWN_TILE(1024)
     nktile::down_rows<IV / 128, false, false, CHOOSE>(hq, hs, w2, w2s, sorted_ids, sorted_expert,    \
                                                     num_valid, partial, T, H, Ktot, Etot, NBC);    \
   }
-NK_DOWN_ROWS(256, 4, true)
-NK_DOWN_ROWS(512, 4, true)
-NK_DOWN_ROWS(1024, 2, false)  // 100 KiB of LDS: one workgroup per CU
+NK_DOWN_ROWS(256, i256, 4, false)
+NK_DOWN_ROWS(256, i256_once, 4, true)
+NK_DOWN_ROWS(512, i512, 4, false)
+NK_DOWN_ROWS(512, i512_once, 4, true)
+NK_DOWN_ROWS(1024, i1024, 2, false)  // 100 KiB of LDS: one workgroup per CU
 
 // The M768 prefill bridge's producer format: W2 in the AITER layout, fp16
 // split-K2 route partials (half 1 starts half_rows rows after half 0).

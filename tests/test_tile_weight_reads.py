@@ -1,22 +1,41 @@
-"""The tile path's choice of weight loads per expert (moe_gemm_lds.hip,
-moe_gemm_tile.hip): at H 2048, I 512 an expert with one block pair (gate/up) or
-one block (down) reads its weights non-temporally. Every token is on the same
-experts (T rows each, and the shared expert), so T moves all of them across the
-edges: one block, two, an absorbed tail of 1 and 16 rows, a pair of its own,
-two pairs with a tail. Bars of the parity tests: the layer output within 2e-2
-of the float64 oracle, bitwise equal on a second launch."""
+"""The tile path's choice of weight loads (moe_gemm_lds.hip, moe_gemm_tile.hip).
+
+CPU: when a call takes the _once kernels, which load the weights of an expert
+with one block non-temporally, by rows per expert and by the size of the
+weights. GPU: those kernels against the ordinary ones (the same arithmetic: bit
+for bit) and the float64 oracle. Every token is on the same experts (T rows
+each, and the shared expert), so T moves all of them across the edges: one
+block, two, an absorbed tail of 1 and 16 rows, a pair of its own, two pairs with
+a tail. Bars of the parity tests: the layer output within 2e-2 of the oracle,
+bitwise equal on a second launch."""
 import numpy as np
 import pytest
 
 from conftest import gpu_available
+from netra_moe import engine
 from netra_moe.config import MoEConfig
+
+
+# (T, H, I, E, K, S) -> whether down reads one-block experts' W2 non-temporally
+@pytest.mark.parametrize("shape,once", [
+    ((300, 2048, 512, 256, 8, 1), True), ((2560, 2048, 512, 256, 8, 1), True), ((2561, 2048, 512, 256, 8, 1), False),
+    ((4096, 2048, 512, 256, 8, 1), False), ((300, 2048, 512, 32, 4, 0), True), ((300, 2048, 512, 31, 4, 0), False),
+    ((1040, 2048, 512, 16, 4, 1), False), ((512, 2048, 512, 8, 2, 1), False), ((300, 512, 256, 256, 8, 0), True),
+    ((300, 512, 256, 16, 2, 0), False), ((512, 512, 256, 64, 4, 1), False), ((300, 4096, 256, 32, 4, 1), True),
+    ((300, 4096, 256, 16, 4, 1), False)])
+def test_down_rule(shape, once):
+    T, H, I, E, K, S = shape
+    cfg = MoEConfig("rule", T=T, H=H, E=E, K=K, I=I, S=S)
+    sym = next(o for o in engine.operations(cfg, "tile") if o["name"] == "moe.down")["symbol"]
+    assert sym == f"netra_moe_down_rows_i{I}{'_once' if once else ''}_gfx950"
 
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
 @pytest.mark.parametrize("T,H,I", [(t, 2048, 512) for t in (64, 65, 128, 129, 144, 145, 257, 272)]
+                         + [(t, h, 256) for h in (512, 4096) for t in (64, 65, 130)]
                          + [(t, 1024, 1024) for t in (300, 700, 2000)])  # I 1024: down_tile, down_rows of 2 and 4 groups
-def test_experts_of_every_block_count(T, H, I):
+def test_experts_of_every_block_count(T, H, I, monkeypatch):
     import torch
 
     import oracle
@@ -28,6 +47,10 @@ def test_experts_of_every_block_count(T, H, I):
     x, gpu_w, host = make_inputs(cfg, dev)
     got = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
     np.testing.assert_array_equal(got["runs"][0], got["runs"][1])
+    monkeypatch.setattr(engine, "weights_once", lambda cfg, expert_bytes: True)
+    once = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
+    np.testing.assert_array_equal(once["runs"][0], once["runs"][1])
+    np.testing.assert_array_equal(once["out"], got["out"])
     ref = oracle_routing(cfg, host)
     np.testing.assert_array_equal(got["topk_ids"], ref["topk_ids"])
     tokens = sample_tokens(cfg, 64)
