@@ -101,9 +101,9 @@
 //       num_valid, pair_map, hq, hs; T, H, I, Ktot, Etot)   H in {512,1024,2048},
 //       grid 8*ceil(CAP*I/128/8), block 512, static LDS <= 155 KiB, T*H < 2^31;
 //       one item per (block pair, 128 h columns), assigned XCD-major
-//   netra_moe_down_rows_i<I>[_once]_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert,
+//   netra_moe_down_rows_i<I>[_cached]_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert,
 //       num_valid, partial bf16[T*Ktot,H]; T, H, I, Ktot, Etot, NBC)   I in {256,512,1024}
-//       (_once, I in {256,512}: an expert with one block reads its W2 non-temporally),
+//       (I in {256,512}: an expert with one block reads its W2 non-temporally; _cached: none does),
 //       grid 8*ceil(CAP*(H/128/NBC)/8), block 512, T*Ktot*H*2 < 2^31; one item per
 //       (64-row block, NBC consecutive 128-column groups), NBC divides H/128
 //   netra_moe_down_tile_i<I>_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert, num_valid,

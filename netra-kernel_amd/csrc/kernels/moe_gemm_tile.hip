@@ -650,7 +650,7 @@ NK_DOWN_TILE(256)
 NK_DOWN_TILE(512)
 NK_DOWN_TILE(1024)
 
-// _once: kChoose (the engine's rule for it: engine.py, weights_once)
+// _cached: without kChoose (the engine's rule for it: engine.py, weights_cached)
 #define NK_DOWN_ROWS(IV, NAME, WPE, CHOOSE)                                                         \
   NK_KERNEL __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE)))                      \
   void netra_moe_down_rows_##NAME##_gfx950(                                                       \
@@ -663,10 +663,10 @@ NK_DOWN_TILE(1024)
     nktile::down_rows<IV / 128, false, false, CHOOSE>(hq, hs, w2, w2s, sorted_ids, sorted_expert,    \
                                                     num_valid, partial, T, H, Ktot, Etot, NBC);    \
   }
-NK_DOWN_ROWS(256, i256, 4, false)
-NK_DOWN_ROWS(256, i256_once, 4, true)
-NK_DOWN_ROWS(512, i512, 4, false)
-NK_DOWN_ROWS(512, i512_once, 4, true)
+NK_DOWN_ROWS(256, i256, 4, true)
+NK_DOWN_ROWS(256, i256_cached, 4, false)
+NK_DOWN_ROWS(512, i512, 4, true)
+NK_DOWN_ROWS(512, i512_cached, 4, false)
 NK_DOWN_ROWS(1024, i1024, 2, false)  // 100 KiB of LDS: one workgroup per CU
 
 // The M768 prefill bridge's producer format: W2 in the AITER layout, fp16

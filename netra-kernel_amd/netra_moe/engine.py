@@ -62,7 +62,7 @@ STREAM_H = (512, 1024, 2048, 4096)   # netra_moe_gate_up_stream_h<H>_c<CH>_gfx95
 STREAM_I = (256, 512, 1024, 2048)    # netra_moe_down_stream_i<I>_c<DC>_gfx950
 TILE_H = (512, 1024, 2048, 4096)     # netra_moe_gate_up_tile_h<H>_gfx950
 TILE_I = (256, 512, 1024)            # netra_moe_down_tile_i<I>_gfx950
-ROWS_I = (256, 512, 1024)            # netra_moe_down_rows_i<I>[_once]_gfx950 (block rows x runs of column groups)
+ROWS_I = (256, 512, 1024)            # netra_moe_down_rows_i<I>[_cached]_gfx950 (block rows x runs of column groups)
 # down_rows: fewer column groups per item until about this many items (I 1024:
 # one workgroup per CU fits and an item stages 64 KiB of rows; down µs at H
 # 1024, E 24, K 3 with 1024 / 256 / 128: T = 600 18.4 / 18.6 / 14.5, 1000 26.5 /
@@ -398,28 +398,28 @@ def _screen_front(cfg: MoEConfig) -> list[dict]:
                    "manifests/gfx950/models/qwen36-35b-c64-fp8.json:43-49"]),
     ]
 
-ONCE_I = (256, 512)                  # netra_moe_down_rows_i<I>_once_gfx950
-# Where a tile-path GEMM takes its _once kernel, which loads the weights of an
-# expert with one block of rows non-temporally. Up to 80 routed rows per expert
-# (T K / E): beyond, most experts have more blocks and only the choice's own
-# loads and branch remain. From 32 MiB of that matrix over all experts (the
-# eight L2 caches together): smaller weights are found in the caches when a
-# call repeats. down us, ordinary / _once, three weight sets in turn (and, in
-# brackets, enough sets that every call reads them from HBM): H 2048, I 512, E
-# 256, K 8, T = 300 62.8 / 56.0, 1000 72.5 / 64.9, 2048 (64 rows) 81.8 / 81.6,
-# 3000 (94) 97.0 / 102; E 128, T = 1000 45.3 / 41.4, 1500 (94) 50.4 / 52.3; E 16
-# (17 MiB), K 4, T = 257 10.0 / 10.4 (11.6 / 10.5), 1040 (260) 21.1 / 21.2; I
-# 256: H 512, E 256 (32 MiB), T = 300 16.7 / 14.1, E 192 11.4 / 11.6 (T = 600
+CACHED_I = (256, 512)                # netra_moe_down_rows_i<I>_cached_gfx950
+# Where a tile-path GEMM takes its _cached kernel; the other one loads the
+# weights of an expert with one block of rows non-temporally. Above so many
+# routed rows per expert (T K / E) most experts have more, and only the
+# choice's own loads and branch remain. Below 32 MiB of that matrix over all
+# experts (the eight L2 caches together) the weights are found in the caches
+# when a call repeats. down us, _cached / the other, three weight sets in turn
+# (and, in brackets, enough sets that every call reads them from HBM): H 2048, I
+# 512, E 256, K 8, T = 300 62.8 / 56.0, 1000 72.5 / 64.9, 2048 (64 rows) 81.8 /
+# 81.6, 3000 (94) 97.0 / 102; E 128, T = 1000 45.3 / 41.4, 1500 (94) 50.4 / 52.3;
+# E 16 (17 MiB), K 4, T = 257 10.0 / 10.4 (11.6 / 10.5), 1040 (260) 21.1 / 21.2;
+# I 256: H 512, E 256 (32 MiB), T = 300 16.7 / 14.1, E 192 11.4 / 11.6 (T = 600
 # 10.8 / 12.0), E 64 6.1 / 6.7, E 16 3.8 / 4.2; H 4096, E 32 18.6 / 16.8, E 16
 # 14.0 / 14.4.
-ONCE_MAX_ROWS = 80
-ONCE_MIN_BYTES = 32 << 20
+CACHED_MIN_ROWS = {"down": 80}
+CACHED_MAX_BYTES = 32 << 20
 
 
-def weights_once(cfg: MoEConfig, expert_bytes: int) -> bool:
-    """Whether a tile-path GEMM with expert_bytes of weights per expert takes
-    its _once kernel."""
-    return cfg.T * cfg.K <= ONCE_MAX_ROWS * cfg.E and cfg.Etot * expert_bytes >= ONCE_MIN_BYTES
+def weights_cached(cfg: MoEConfig, op: str) -> bool:
+    """Whether a tile-path GEMM takes its _cached kernel."""
+    expert_bytes = cfg.H * cfg.I
+    return cfg.T * cfg.K > CACHED_MIN_ROWS[op] * cfg.E or cfg.Etot * expert_bytes < CACHED_MAX_BYTES
 
 
 def down_rows_groups(cfg: MoEConfig) -> int:
@@ -649,8 +649,8 @@ def _tile_down(cfg: MoEConfig) -> dict:
     # (I 1024 at one group per item: the 64 KiB of rows are staged for one
     # group, no faster than down_tile: T = 300, E 24, K 3 11.8 / 11.7 us)
     if I in ROWS_I and (I < 1024 or nbc > 1) and cfg.routes * H * 2 < 1 << 31:
-        once = "_once" if I in ONCE_I and weights_once(cfg, H * I) else ""
-        return dict(name="moe.down", symbol=f"netra_moe_down_rows_i{I}{once}_gfx950",
+        cached = "_cached" if I in CACHED_I and weights_cached(cfg, "down") else ""
+        return dict(name="moe.down", symbol=f"netra_moe_down_rows_i{I}{cached}_gfx950",
                     grid=(xcd_grid(cfg.cap_blocks * (H // 128 // nbc)), 1, 1), block=(512, 1, 1),
                     lds=64 * I + 2 * 64 * 272 + 64 * (I // 128) * 4 + 64 * 4, dyn=0,
                     args=["h_q", "h_scale", "w2", "w2_scale", *common, "partial",

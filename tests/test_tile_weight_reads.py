@@ -1,8 +1,8 @@
 """The tile path's choice of weight loads (moe_gemm_lds.hip, moe_gemm_tile.hip).
 
-CPU: when a call takes the _once kernels, which load the weights of an expert
-with one block non-temporally, by rows per expert and by the size of the
-weights. GPU: those kernels against the ordinary ones (the same arithmetic: bit
+CPU: when a call takes the _cached kernels, by rows per expert and by the size
+of the weights; the others load the weights of an expert with one block
+non-temporally. GPU: those against the _cached ones (the same arithmetic: bit
 for bit) and the float64 oracle. Every token is on the same experts (T rows
 each, and the shared expert), so T moves all of them across the edges: one
 block, two, an absorbed tail of 1 and 16 rows, a pair of its own, two pairs with
@@ -17,17 +17,17 @@ from netra_moe.config import MoEConfig
 
 
 # (T, H, I, E, K, S) -> whether down reads one-block experts' W2 non-temporally
-@pytest.mark.parametrize("shape,once", [
+@pytest.mark.parametrize("shape,chooses", [
     ((300, 2048, 512, 256, 8, 1), True), ((2560, 2048, 512, 256, 8, 1), True), ((2561, 2048, 512, 256, 8, 1), False),
     ((4096, 2048, 512, 256, 8, 1), False), ((300, 2048, 512, 32, 4, 0), True), ((300, 2048, 512, 31, 4, 0), False),
     ((1040, 2048, 512, 16, 4, 1), False), ((512, 2048, 512, 8, 2, 1), False), ((300, 512, 256, 256, 8, 0), True),
     ((300, 512, 256, 16, 2, 0), False), ((512, 512, 256, 64, 4, 1), False), ((300, 4096, 256, 32, 4, 1), True),
     ((300, 4096, 256, 16, 4, 1), False)])
-def test_down_rule(shape, once):
+def test_down_rule(shape, chooses):
     T, H, I, E, K, S = shape
     cfg = MoEConfig("rule", T=T, H=H, E=E, K=K, I=I, S=S)
     sym = next(o for o in engine.operations(cfg, "tile") if o["name"] == "moe.down")["symbol"]
-    assert sym == f"netra_moe_down_rows_i{I}{'_once' if once else ''}_gfx950"
+    assert sym == f"netra_moe_down_rows_i{I}{'' if chooses else '_cached'}_gfx950"
 
 
 @pytest.mark.gpu
@@ -45,12 +45,13 @@ def test_experts_of_every_block_count(T, H, I, monkeypatch):
     print(f"\n[reads] {cfg}", flush=True)
     dev = torch.device("cuda", 0)
     x, gpu_w, host = make_inputs(cfg, dev)
+    assert engine.weights_cached(cfg, "down")
+    cached = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
+    np.testing.assert_array_equal(cached["runs"][0], cached["runs"][1])
+    monkeypatch.setattr(engine, "weights_cached", lambda cfg, op: False)
     got = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
     np.testing.assert_array_equal(got["runs"][0], got["runs"][1])
-    monkeypatch.setattr(engine, "weights_once", lambda cfg, expert_bytes: True)
-    once = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
-    np.testing.assert_array_equal(once["runs"][0], once["runs"][1])
-    np.testing.assert_array_equal(once["out"], got["out"])
+    np.testing.assert_array_equal(cached["out"], got["out"])
     ref = oracle_routing(cfg, host)
     np.testing.assert_array_equal(got["topk_ids"], ref["topk_ids"])
     tokens = sample_tokens(cfg, 64)
