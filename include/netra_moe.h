@@ -97,10 +97,11 @@
 //   netra_moe_gate_up_tile_h<H>_gfx950(xq, xs, w13, w13s, sorted_ids, sorted_expert,
 //       num_valid, hq e4m3[CAP*64,I], hs f32[CAP*64,I/128]; T, H, I, Ktot, Etot)
 //       grid 8*ceil(CAP*I/128/8), block 256 (items assigned XCD-major); used for H = 4096
-//   netra_moe_gate_up_lds_h<H>_gfx950(xq, xs, w13, w13s, sorted_ids, sorted_expert,
+//   netra_moe_gate_up_lds_h<H>[_cached]_gfx950(xq, xs, w13, w13s, sorted_ids, sorted_expert,
 //       num_valid, pair_map, hq, hs; T, H, I, Ktot, Etot)   H in {512,1024,2048},
 //       grid 8*ceil(CAP*I/128/8), block 512, static LDS <= 155 KiB, T*H < 2^31;
-//       one item per (block pair, 128 h columns), assigned XCD-major
+//       one item per (block pair, 128 h columns), assigned XCD-major (H 2048: an
+//       expert with one pair reads its W13 non-temporally; _cached, H 2048: none does)
 //   netra_moe_down_rows_i<I>[_cached]_gfx950(hq, hs, w2, w2s, sorted_ids, sorted_expert,
 //       num_valid, partial bf16[T*Ktot,H]; T, H, I, Ktot, Etot, NBC)   I in {256,512,1024}
 //       (I in {256,512}: an expert with one block reads its W2 non-temporally; _cached: none does),

@@ -93,7 +93,7 @@ __device__ __forceinline__ void copy16(uint32_t m0, u32x4 r, uint32_t voff, uint
                : "memory");
 }
 
-// copy16 with a non-temporal load, for weights a launch reads about once.
+// copy16 with a non-temporal load, for weights that one item of a launch reads.
 __device__ __forceinline__ void copy16_once(uint32_t m0, u32x4 r, uint32_t voff, uint32_t soff) {
   uint32_t saved;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds\n\t"
@@ -164,15 +164,18 @@ __device__ __forceinline__ bool xcd_item(uint32_t i, uint32_t n, uint32_t& item)
 // rows I..2I-1 as plain row tiles) instead of the gate/up-interleaved
 // tile16x128 layout; the copies move the same 2 KiB blocks, only the up tile's
 // place and the operand reads out of LDS differ.
-// kChoose: an item whose expert has no other block pair copies W13 with
-// non-temporal loads (no other item reads that slice, and its lines leave the
-// activations in the L2); with more pairs the copies are ordinary, and the
-// pairs' items find each other's lines there. gate/up us at H 2048, I 512, E
-// 256, K 8, all ordinary / all non-temporal / chosen: T = 512 113.1 / 107.0 /
-// 106.0, 1000 115.9 / 110.9 / 108.9, 2048 121.7 / 119.6 / 119.1, 4096 145.4 /
-// 149.8 / 145.4; Zipf-skewed 512 46.2 / 43.3 / 41.1, 1000 60.8 / 61.0 / 56.9,
-// 4096 140.1 / 147.7 / 137.2. (H 1024, whose tens of MB of weights the caches
-// hold: 39.4 / 44.2 at T = 2000, E 24, so only H 2048 chooses.)
+// kChoose: an item whose expert has no other block pair (a tail that it
+// absorbs is not one) copies W13 with non-temporal loads (no other item reads
+// that slice, and its lines leave the activations in the L2); with more pairs
+// the copies are ordinary, and the pairs' items find each other's lines
+// there. gate/up us at H 2048, I 512, E 256, K 8, all ordinary / all
+// non-temporal / chosen: T = 512 113.1 / 107.0 / 106.0, 1000 115.9 / 110.9 /
+// 108.9, 2048 121.7 / 119.6 / 119.1, 4096 145.4 / 149.8 / 145.4; Zipf-skewed
+// 512 46.2 / 43.3 / 41.1, 1000 60.8 / 61.0 / 56.9, 4096 140.1 / 147.7 / 137.2.
+// The K loop is there once for each kind of copy: a branch in every copy
+// measured 62.7 against 60.4 (Zipf T = 1000). (H 1024, whose tens of MB of
+// weights the caches hold: 39.4 / 44.2 at T = 2000, E 24, so only H 2048 has
+// the choice.)
 template <uint32_t KB, bool kAiter = false, bool kChoose = false>  // H / 128
 __device__ __forceinline__ void gate_up_lds(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13,
@@ -340,6 +343,14 @@ __device__ __forceinline__ void gate_up_lds(
       if (kb == 0) wsv = s_wsv[lane];  // the scale copy landed with step 0's copies
       if (NT > 0) {
         const uint8_t* st = s_stage[kb % kStages];
+        // (kChoose: opaque every four K blocks. Kept for the whole loop, the
+        // scales' addresses took the last of 256 registers and one was spilled:
+        // 8 bytes of scratch for every launch.)
+        uint32_t row = 0u;
+        if constexpr (kChoose) {
+          row = lane & 15u;
+          if (kb % 4u == 0u) asm volatile("" : "+v"(row));
+        }
         v8i bw[4];
 #pragma unroll
         for (uint32_t c = 0; c < 4; ++c)  // gate tiles 2n, 2n + 1, up tiles 8 + 2n, 8 + 2n + 1
@@ -350,7 +361,7 @@ __device__ __forceinline__ void gate_up_lds(
         for (uint32_t i = 0; i < NT; ++i) {
           const uint32_t rt = 4u * m + i;
           const v8i af = lds_operand_rows(st + rt * 2048u, lane);
-          const float as = s_as_at(rt * 16u + (lane & 15u), kb);  // this lane's token row
+          const float as = s_as_at(rt * 16u + (kChoose ? row : lane & 15u), kb);  // this lane's token row
           const float sgi = sg * as, sui = su * as;
           some_copies(i + 1u < NT ? kPer : kCopies);
           v4f d[4];
@@ -390,13 +401,15 @@ __device__ __forceinline__ void gate_up_lds(
       default: kloop(std::integral_constant<uint32_t, 4>{}, no_tail{}, oncec); break;
     }
   };
-  // kChoose: whether this item alone reads its W13 slice (the expert has no
-  // other pair; an absorbed tail ends it)
-  const bool alone = kChoose && ep != e && (!two || e3 != e);
-  if (absorb) {
-    kloop(std::integral_constant<uint32_t, 4>{}, std::true_type{}, std::integral_constant<bool, kChoose>{});
-  } else if (alone) {  // uniform
-    by_tiles(std::integral_constant<bool, kChoose>{});
+  // kChoose: whether no other item reads this item's W13 slice (no other pair
+  // before it, and behind it at most the tail that it absorbs)
+  using once = std::integral_constant<bool, kChoose>;
+  const bool alone = kChoose && ep != e && (!two || e3 != e || absorb);
+  if (absorb) {  // (all uniform)
+    if (alone) kloop(std::integral_constant<uint32_t, 4>{}, std::true_type{}, once{});
+    else kloop(std::integral_constant<uint32_t, 4>{}, std::true_type{}, std::false_type{});
+  } else if (alone) {
+    by_tiles(once{});
   } else {
     by_tiles(std::false_type{});
   }
@@ -486,8 +499,9 @@ __device__ __forceinline__ void gate_up_lds(
 }
 }  // namespace nklds
 
-#define NK_GATE_UP_LDS(HV, CHOOSE)                                                                 \
-  NK_KERNEL __launch_bounds__(512) void netra_moe_gate_up_lds_h##HV##_gfx950(                      \
+// _cached: without kChoose (the engine's rule for it: engine.py, weights_cached)
+#define NK_GATE_UP_LDS(HV, NAME, CHOOSE)                                                           \
+  NK_KERNEL __launch_bounds__(512) void netra_moe_gate_up_lds_##NAME##_gfx950(                     \
       const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13, \
       const float* __restrict__ w13s, const int32_t* __restrict__ sorted_ids,                      \
       const int32_t* __restrict__ sorted_expert, const int32_t* __restrict__ num_valid,            \
@@ -497,9 +511,10 @@ __device__ __forceinline__ void gate_up_lds(
     nklds::gate_up_lds<HV / 128, false, CHOOSE>(xq, xs, w13, w13s, sorted_ids, sorted_expert,      \
                                                 num_valid, pair_map, hq, hs, T, I, Ktot, Etot);    \
   }
-NK_GATE_UP_LDS(512, false)
-NK_GATE_UP_LDS(1024, false)
-NK_GATE_UP_LDS(2048, true)
+NK_GATE_UP_LDS(512, h512, false)
+NK_GATE_UP_LDS(1024, h1024, false)
+NK_GATE_UP_LDS(2048, h2048, true)
+NK_GATE_UP_LDS(2048, h2048_cached, false)
 
 // W13 in the reference's AITER layout (the M768 prefill bridge): same ABI.
 #define NK_GATE_UP_LDS_AITER(HV)                                                                   \

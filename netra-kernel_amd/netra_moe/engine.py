@@ -71,7 +71,7 @@ ROWS_I = (256, 512, 1024)            # netra_moe_down_rows_i<I>[_cached]_gfx950 
 DOWN_ROWS_ITEMS = {256: 1024, 512: 1024, 1024: 128}
 TILE_GU_WAVES = 4                    # waves of netra_moe_gate_up_tile_h<H>_gfx950 (its launch bound)
 SPLIT_HI = ((2048, 512),)            # netra_moe_gate_up_split_h<H>_{tiles|rows}_gfx950
-LDS_GU_H = (512, 1024, 2048)         # netra_moe_gate_up_lds_h<H>_gfx950: 128-row pairs, LDS operand ring
+LDS_GU_H = (512, 1024, 2048)         # netra_moe_gate_up_lds_h<H>[_cached]_gfx950: 128-row pairs, LDS operand ring
 # Stream kernel grids (measured at T=64 on one MI355X): gate/up fills the chip
 # once, 256 CUs x 4 SIMDs x 2 resident waves (NK_GATE_UP_WAVES_PER_EU) / 8
 # waves per workgroup; down runs 4096 four-wave workgroups, about four times
@@ -399,26 +399,33 @@ def _screen_front(cfg: MoEConfig) -> list[dict]:
     ]
 
 CACHED_I = (256, 512)                # netra_moe_down_rows_i<I>_cached_gfx950
+CACHED_H = (2048,)                   # netra_moe_gate_up_lds_h<H>_cached_gfx950
 # Where a tile-path GEMM takes its _cached kernel; the other one loads the
-# weights of an expert with one block of rows non-temporally. Above so many
-# routed rows per expert (T K / E) most experts have more, and only the
-# choice's own loads and branch remain. Below 32 MiB of that matrix over all
-# experts (the eight L2 caches together) the weights are found in the caches
-# when a call repeats. down us, _cached / the other, three weight sets in turn
-# (and, in brackets, enough sets that every call reads them from HBM): H 2048, I
-# 512, E 256, K 8, T = 300 62.8 / 56.0, 1000 72.5 / 64.9, 2048 (64 rows) 81.8 /
-# 81.6, 3000 (94) 97.0 / 102; E 128, T = 1000 45.3 / 41.4, 1500 (94) 50.4 / 52.3;
-# E 16 (17 MiB), K 4, T = 257 10.0 / 10.4 (11.6 / 10.5), 1040 (260) 21.1 / 21.2;
-# I 256: H 512, E 256 (32 MiB), T = 300 16.7 / 14.1, E 192 11.4 / 11.6 (T = 600
-# 10.8 / 12.0), E 64 6.1 / 6.7, E 16 3.8 / 4.2; H 4096, E 32 18.6 / 16.8, E 16
-# 14.0 / 14.4.
-CACHED_MIN_ROWS = {"down": 80}
+# weights of an expert with one block of rows (gate/up: one 128-row pair)
+# non-temporally. Above so many routed rows per expert (T K / E) most experts
+# have more, and only the choice's own cost remains. Below 32 MiB of that matrix
+# over all experts (the eight L2 caches together) the weights are found in the
+# caches when a call repeats. us, _cached / the other, three weight sets in turn
+# (in brackets: enough sets that every call reads them from HBM).
+# gate/up at H 2048, I 512: E 256, K 8, T = 300 109.4 / 105.0, 1000 114.9 /
+# 109.3, 2048 119.8 / 116.9, 3000 (94 rows) 127.3 / 122.7; layer T = 4096 (128)
+# 302.3 / 299.8; Zipf-skewed 512 47.5 / 43.2, 1000 64.4 / 60.4, 2048 84.4 / 81.2;
+# E 64, K 4, T = 1000 44.4 / 41.2, layer T = 2048 (128) 121.1 / 121.5, 4096 (256)
+# 175.2 / 177.9; E 32, T = 300 20.3 / 20.5 (23.3 / 20.7), 2048 (256) 42.4 / 43.6;
+# E 8 (18 MiB), K 2, T = 512 21.3 / 22.1.
+# down: H 2048, I 512, E 256, K 8, T = 300 62.8 / 56.0, 1000 72.5 / 64.9, 2048
+# (64 rows) 81.8 / 81.6, 3000 (94) 97.0 / 102; E 128, T = 1000 45.3 / 41.4, 1500
+# (94) 50.4 / 52.3; E 16 (17 MiB), K 4, T = 257 10.0 / 10.4 (11.6 / 10.5), 1040
+# (260) 21.1 / 21.2; I 256: H 512, E 256 (32 MiB), T = 300 16.7 / 14.1, E 192
+# 11.4 / 11.6 (T = 600 10.8 / 12.0), E 64 6.1 / 6.7, E 16 3.8 / 4.2; H 4096, E
+# 32 18.6 / 16.8, E 16 14.0 / 14.4.
+CACHED_MIN_ROWS = {"gate_up": 128, "down": 80}
 CACHED_MAX_BYTES = 32 << 20
 
 
 def weights_cached(cfg: MoEConfig, op: str) -> bool:
-    """Whether a tile-path GEMM takes its _cached kernel."""
-    expert_bytes = cfg.H * cfg.I
+    """Whether a tile-path GEMM (gate_up or down) takes its _cached kernel."""
+    expert_bytes = cfg.H * cfg.I * (2 if op == "gate_up" else 1)
     return cfg.T * cfg.K > CACHED_MIN_ROWS[op] * cfg.E or cfg.Etot * expert_bytes < CACHED_MAX_BYTES
 
 
@@ -711,8 +718,9 @@ def operations(cfg: MoEConfig, path: str = "auto", front: str = "auto") -> list[
         if H in LDS_GU_H:
             if T * H >= 1 << 31:
                 raise ValueError("netra_moe_gate_up_lds needs T * H < 2^31 (32-bit activation offsets)")
+            cached = "_cached" if H in CACHED_H and weights_cached(cfg, "gate_up") else ""
             gate_up = dict(
-                name="moe.gate_up", symbol=f"netra_moe_gate_up_lds_h{H}_gfx950",
+                name="moe.gate_up", symbol=f"netra_moe_gate_up_lds_h{H}{cached}_gfx950",
                 grid=(xcd_grid(cfg.cap_blocks * (I // 128)), 1, 1), block=(512, 1, 1),
                 lds=gate_up_lds_bytes(H), dyn=0,
                 args=["x_q", "x_scale", "w13", "w13_scale", *common, "pair_map", "h_q", "h_scale",

@@ -34,7 +34,7 @@ def scratch_bytes(artefact, tmp_path) -> dict[str, int]:
     return {one(k, "name"): int(one(k, "private_segment_fixed_size")) for k in kernels}
 
 
-@pytest.mark.parametrize("family", ["down", "ffn", "combine"])
+@pytest.mark.parametrize("family", ["gate_up", "down", "ffn", "combine"])
 @pytest.mark.parametrize("artefact", sorted(ARTEFACTS))
 def test_gemm_kernels_need_no_scratch(artefact, family, tmp_path):
     found = {n: b for n, b in scratch_bytes(artefact, tmp_path).items()

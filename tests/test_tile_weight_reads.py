@@ -2,11 +2,11 @@
 
 CPU: when a call takes the _cached kernels, by rows per expert and by the size
 of the weights; the others load the weights of an expert with one block
-non-temporally. GPU: those against the _cached ones (the same arithmetic: bit
-for bit) and the float64 oracle. Every token is on the same experts (T rows
-each, and the shared expert), so T moves all of them across the edges: one
-block, two, an absorbed tail of 1 and 16 rows, a pair of its own, two pairs with
-a tail. Bars of the parity tests: the layer output within 2e-2 of the oracle,
+(gate/up: one block pair) non-temporally. GPU: those against the _cached ones
+(the same arithmetic: bit for bit) and the float64 oracle. Every token is on the
+same experts (T rows each, and the shared expert), so T moves all of them across
+the edges: one block, two, an absorbed tail of 1 and 16 rows, a pair of its own,
+two pairs with a tail. Bars of the parity tests: the layer output within 2e-2 of the oracle,
 bitwise equal on a second launch."""
 import numpy as np
 import pytest
@@ -14,6 +14,17 @@ import pytest
 from conftest import gpu_available
 from netra_moe import engine
 from netra_moe.config import MoEConfig
+
+
+# (T, H, I, E, K, S) -> whether gate/up reads one-pair experts' W13 non-temporally
+@pytest.mark.parametrize("shape,chooses", [
+    ((512, 2048, 512, 256, 8, 1), True), ((4096, 2048, 512, 256, 8, 1), True), ((4097, 2048, 512, 256, 8, 1), False),
+    ((1040, 2048, 512, 16, 4, 1), False), ((512, 2048, 512, 8, 2, 1), False), ((300, 2048, 512, 16, 4, 0), True)])
+def test_gate_up_rule(shape, chooses):
+    T, H, I, E, K, S = shape
+    cfg = MoEConfig("rule", T=T, H=H, E=E, K=K, I=I, S=S)
+    sym = next(o for o in engine.operations(cfg, "tile") if o["name"] == "moe.gate_up")["symbol"]
+    assert sym == f"netra_moe_gate_up_lds_h{H}{'' if chooses else '_cached'}_gfx950"
 
 
 # (T, H, I, E, K, S) -> whether down reads one-block experts' W2 non-temporally
@@ -45,7 +56,7 @@ def test_experts_of_every_block_count(T, H, I, monkeypatch):
     print(f"\n[reads] {cfg}", flush=True)
     dev = torch.device("cuda", 0)
     x, gpu_w, host = make_inputs(cfg, dev)
-    assert engine.weights_cached(cfg, "down")
+    assert engine.weights_cached(cfg, "down") and engine.weights_cached(cfg, "gate_up")
     cached = run_gpu(cfg, x, gpu_w, dev, expose=("topk_ids",), repeats=2, path="tile")
     np.testing.assert_array_equal(cached["runs"][0], cached["runs"][1])
     monkeypatch.setattr(engine, "weights_cached", lambda cfg, op: False)
