@@ -89,7 +89,7 @@
 //       w2s f32[Etot,H/128,I/128], sorted_ids, sorted_expert, tile_map, num_valid,
 //       partial f32[T*Ktot,H]; T, H, I, Ktot, Etot)   grid 2048, block 256
 //       (DC K blocks per step, 1 or 2)
-//   few rows per expert (T * K <= 13 E), H = 2048, I = 512:
+//   few rows per expert (at most 13 E routed rows, T * K), H = 2048, I = 512:
 //   netra_moe_gate_up_split_h2048_<tiles|rows>_gfx950(xq, xs, w13, w13s, sorted_ids, counts,
 //       hq, hs; T, I, Etot, CAP)   grid 256, block 512, static LDS 149 KiB, T*H < 2^31, CAP <
 //       65536; hq / hs as gate_up_stream's (tiles) or gate_up_lds' (rows)

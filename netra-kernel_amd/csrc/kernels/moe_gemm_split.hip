@@ -16,10 +16,10 @@
 // 82.2, 100 93.2 / 84.6, 128 112.8 / 89.3, 192 115.3 / 98, 256 120.9 / 100
 // (stream); T = 257 109.2 / 93.5, 400 110.8 / 96.3 (block pairs). Skewed
 // routing (Zipf 1.1): T = 100 33.6 / 28.0, 192 52.1 / 45.4, 400 46.8 / 42.8,
-// but 512 46.0 / 53.0: an expert of hundreds of rows is many chunks here, each
-// with a K-split sum per 64 rows, and the block pairs serve it better; at 16
-// rows per expert (T = 512) and above they keep the call (uniform routing
-// there: 111 / 96).
+// but 512 46.0 / 53.0 (uniform routing there: 111 / 96): an expert of hundreds
+// of rows is many chunks here, each with a K-split sum per 64 rows, and the
+// block pairs serve it better. The engine's rule (engine.py, split_gate_up)
+// ends at 13 routed rows per expert, and leaves few-row calls to the others.
 //
 //   netra_moe_gate_up_split_h<H>_{tiles|rows}_gfx950(xq, xs, w13, w13s,
 //       sorted_ids, counts, hq, hs; T, I, Etot, CAP)   grid 256, block 512

@@ -146,18 +146,42 @@ def xcd_grid(items: int) -> int:
 
 
 SPLIT_GRID = 256                     # one workgroup per CU
-# Rows per routed expert (T K / E) up to which gate/up is the split kernel.
-# Gate/up times, µs, the path's other kernel / split: T = 80
-# (2.5 rows) 88.1 / 82.2, 192 (6) 115.3 / 98, 400 (12.5) 110.8 / 96.3; with
-# Zipf-skewed routing T = 192 52.1 / 45.4, 400 46.8 / 42.8, 512 (16) 46.0 /
-# 53.0 (uniform at 512: 111 / 96). T = 65 84.3 / 83.6.
-SPLIT_MAX_ROWS = 13
+# Where gate/up is the split kernel. It deals 128-column blocks of h, a whole
+# number to every workgroup, so its time goes in rounds of 256 blocks (about 20
+# us each), the last one whole however few blocks are left for it; it has no
+# advantage with tens of row tiles, or once the rows of an expert fill several
+# of its 64-row chunks. Layer times, us, with the path's other gate/up / split,
+# uniform routing; Zipf-skewed routing:
+#   stream path, S 1, K 8 unless said. E 256: T = 65 144.6 / 144.8; 65.7 / 58.3,
+#   100 164.5 / 161.0; 74.3 / 65.0, 192 198.8 / 187.5; 102.9 / 95.3. E 512, K 10:
+#   T = 65 242 / 231; 79.5 / 72.9, 256 361 / 347; 141 / 123. With a poorly filled
+#   last round the uniform calls lose what the skewed ones gain, and less: E 64,
+#   T = 104 68.5 / 75.4; 68.1 / 59.3, E 128, T = 128 105 / 111; 74.2 / 64.8, E 160
+#   120 / 128; 76.4 / 67.2, E 224 155 / 160; 80.7 / 73.2, E 128, K 4, T = 140 104 /
+#   106; 58.6 / 54.6. Fewer than about 512 routed rows lose both ways: E 256, K 4,
+#   T = 100 138 / 144; 49.2 / 54.6, 128 151 / 152; 53.1 / 57.1, E 64, T = 128 65.8 /
+#   73.9; 48.6 / 50.8, E 32, T = 100 49.3 / 50.6, T = 80 skewed 41.2 / 46.6, E 16, K
+#   2, T = 100 34.0 / 43.4; 33.3 / 43.2.
+#   tile path, E 256, K 8: T = 300 187 / 177; 91.5 / 93.8, 416 190 / 181; 97.2 /
+#   97.8. Fewer rows: E 192, K 6, T = 300 153 / 143; 75.2 / 87.8, E 256, K 4, T =
+#   400 185 / 175; 67.0 / 72.5, K 2, T = 1000 191 / 179; 74.1 / 90.8. E 512, K 10, T
+#   = 400 323 / 315; 109 / 118. T = 512, E 256, K 8, gate/up 111 / 96; 46 / 53.
+SPLIT_MAX_ROWS = 13                  # routed rows per expert (T K / E)
+SPLIT_MAX_T = 416                    # (no expert has more rows than tokens)
+SPLIT_MIN_ROUTES = {"stream": 513, "tile": 2048}
+SPLIT_TILE_MAX_E = 256
+
+
+def split_supported(cfg: MoEConfig, path: str) -> bool:
+    """Whether the split gate/up can serve the stream or tile path's call."""
+    return (path in ("stream", "tile") and (cfg.H, cfg.I) in SPLIT_HI and cfg.T * cfg.H < 1 << 31
+            and cfg.T * cfg.K <= SPLIT_MAX_ROWS * cfg.E and cfg.cap_blocks < 1 << 16)
 
 
 def split_gate_up(cfg: MoEConfig, path: str) -> bool:
     """Whether the stream or tile path's gate/up is the split kernel."""
-    return (path in ("stream", "tile") and (cfg.H, cfg.I) in SPLIT_HI and cfg.T * cfg.H < 1 << 31
-            and cfg.T * cfg.K <= SPLIT_MAX_ROWS * cfg.E and cfg.cap_blocks < 1 << 16)
+    return (split_supported(cfg, path) and cfg.T <= SPLIT_MAX_T and cfg.T * cfg.K >= SPLIT_MIN_ROUTES[path]
+            and (path == "stream" or cfg.E <= SPLIT_TILE_MAX_E))
 
 
 def split_lds_bytes() -> int:

@@ -68,6 +68,20 @@ def test_rule_by_rows_per_expert(T, E, K, path, split):
     assert ("split" in sym) == split
 
 
+# Calls that it slows (both ways, or more by skewed routing than it gains by uniform), and their neighbours
+@pytest.mark.parametrize("T,E,K,S,path,split", [
+    (80, 8, 1, 1, "stream", False), (100, 16, 2, 1, "stream", False), (100, 32, 4, 1, "stream", False),
+    (128, 64, 4, 1, "stream", False), (100, 256, 4, 1, "stream", False), (128, 256, 4, 1, "stream", False),
+    (129, 256, 4, 1, "stream", True), (65, 64, 8, 1, "stream", True), (128, 128, 8, 1, "stream", True),
+    (65, 512, 10, 1, "stream", True), (256, 512, 10, 1, "stream", True), (65, 256, 8, 1, "stream", True),
+    (256, 256, 8, 1, "stream", True), (257, 256, 8, 1, "tile", True), (416, 256, 8, 1, "tile", True),
+    (400, 256, 4, 1, "tile", False), (1000, 256, 2, 1, "tile", False), (3000, 256, 1, 1, "tile", False),
+    (300, 192, 6, 1, "tile", False), (416, 512, 10, 1, "tile", False)])
+def test_rule_by_rows(T, E, K, S, path, split):
+    cfg = MoEConfig("rule", T=T, H=2048, E=E, K=K, I=512, S=S)
+    assert engine.split_gate_up(cfg, path) == split
+
+
 GPU_CASES = {
     "t65": (dict(T=65, E=256, K=8, S=1), "stream"),
     "t1": (dict(T=1, E=256, K=8, S=1), "stream"),
@@ -77,6 +91,7 @@ GPU_CASES = {
     "t65_hot": (dict(T=65, E=256, K=8, S=1, router_bias="hot"), "stream"),
     "t129_hot": (dict(T=129, E=128, K=4, S=1, router_bias="hot"), "tile"),
     "t40_e500": (dict(T=40, E=500, K=12, S=1), "tile"),
+    "t70_e512": (dict(T=70, E=512, K=10, S=1), "stream"),
     "t333_zipf": (dict(T=333, E=256, K=8, S=1, router_bias="zipf1.1"), "tile"),
 }
 
@@ -96,8 +111,10 @@ def test_against_the_general_kernels_and_the_oracle(name, monkeypatch):
     dev = torch.device("cuda", 0)
     x, gpu_w, host = make_inputs(cfg, dev)
     expose = ("topk_ids", "sorted_ids", "h_q", "h_scale")
-    assert engine.split_gate_up(cfg, path)
-    got = run_gpu(cfg, x, gpu_w, dev, expose=expose, repeats=2, path=path)
+    assert engine.split_supported(cfg, path)  # whether or not the rule would take it
+    with monkeypatch.context() as m:
+        m.setattr(engine, "split_gate_up", lambda cfg, path: True)
+        got = run_gpu(cfg, x, gpu_w, dev, expose=expose, repeats=2, path=path)
     with monkeypatch.context() as m:
         m.setattr(engine, "split_gate_up", lambda cfg, path: False)
         gen = run_gpu(cfg, x, gpu_w, dev, expose=expose, path=path)
