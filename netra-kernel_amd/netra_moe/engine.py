@@ -527,10 +527,11 @@ MERGED_KSPLIT_MIN_TILES = {(2048, 512): 150}
 
 
 def expected_tiles(cfg: MoEConfig) -> float:
-    """16-row tiles of a decode call under uniform routing: the routed experts
-    a call is expected to touch, plus the shared experts' tiles."""
-    touched = cfg.E * (1.0 - (1.0 - cfg.K / cfg.E) ** cfg.T) if cfg.E else 0.0
-    return touched + cfg.S * ((cfg.T + 15) // 16)
+    """16-row tiles of a decode call under uniform routing: each routed expert's
+    rows, binomial (T, K / E), in tiles of 16, plus the shared experts' tiles."""
+    T, p = cfg.T, cfg.K / cfg.E
+    routed = sum(math.comb(T, n) * p ** n * (1.0 - p) ** (T - n) * ((n + 15) // 16) for n in range(1, T + 1))
+    return cfg.E * routed + cfg.S * ((T + 15) // 16)
 
 
 def down_variant(cfg: MoEConfig) -> str:
@@ -558,16 +559,19 @@ def ffn_wide_p(cfg: MoEConfig) -> int:
     """Column items per wave of the wide gate/up: a workgroup streams P
     128-column blocks of a tile, so the full P leaves most CUs idle when a call
     has few tiles, and a smaller one costs rounds when it has many. A smaller P
-    is taken where it at least halves rounds x P (the expected items with 6%
-    for the spread of the routing, over 256 workgroups), the larger of equals.
-    Gate/up µs, full / chosen: H 1024, I 1024, E 24, K 3, T = 20 26.0 / 13.1, 40
-    26.8 / 14.1, 64 27.5 / 14.9; H 4096, I 256, E 32, K 4, T = 20 44.9 / 27.7, 64
-    47.1 / 29.2; H 2048, I 512, E 256, K 8, T = 17 (108 tiles) 49.7 / 43.1, 19
-    (118) 54.1 / 48.3, and at 21 (127, where it would cost a second round of P
-    = 2 or a third of 1) 54.6 / 63.3 and 56.3."""
+    is taken where it at least halves rounds x P (the expected items with 4.5%
+    for the spread of the routing, at most every expert with all T rows, over
+    256 workgroups), the larger of equals. Gate/up µs, full / chosen: H 1024, I 1024, E 24, K 3, T = 20
+    26.0 / 13.1, 40 26.8 / 14.1, 64 27.5 / 14.9; E 24, K 8, T = 40 (30 tiles) 27.9 /
+    15.3, 64 (50, P = 2; P = 1 runs a second round: 22.8) 30.1 / 20.6; H 4096, I
+    256, E 32, K 4, T = 20 44.9 / 27.7, 64 47.1 / 29.2; H 2048, I 512, E 16, K 15,
+    T = 60 (64 tiles) 45.5 / 22.9, E 32, K 12 (P = 2; P = 1 39.4) 47.1 / 32.1; E
+    256, K 8, T = 17 (108 tiles) 49.7 / 43.1, 20 (122) 50.5 / 46.7, and at 21 (127,
+    where it would cost a second round of P = 2 or a third of 1) 54.6 / 63.3 and
+    56.3; with K 4, T = 40 (123) 51.4 / 53.9."""
     full = FFN_WIDE_P[(cfg.H, cfg.I)]
-    tiles, blocks = expected_tiles(cfg), cfg.I // 128
-    cost = lambda p: math.ceil(1.06 * tiles * (blocks // p) / FFN_GRID[("gate_up", "wide")]) * p  # noqa: E731
+    tiles, blocks = min(1.045 * expected_tiles(cfg), cfg.Etot * ((cfg.T + 15) // 16)), cfg.I // 128
+    cost = lambda p: math.ceil(tiles * (blocks // p) / FFN_GRID[("gate_up", "wide")]) * p  # noqa: E731
     best = min(FFN_SPREAD_P.get((cfg.H, cfg.I), ()), key=lambda p: (cost(p), -p), default=full)
     return best if 2 * cost(best) <= cost(full) else full
 

@@ -245,8 +245,8 @@ def test_op_bridges_declare_the_reference_bridge_abis():
 def test_merged_decode_ffn_follows_the_expected_tile_count():
     """The fused path merges each tile's down into gate/up only when a call is
     expected to have enough 16-row tiles to keep the chip streaming (the
-    expected count under uniform routing: E (1 - (1 - K/E)^T) + S ceil(T/16),
-    checked against a direct sum over experts), and splits gate/up's K over
+    expected count under uniform routing; with few rows per expert E (1 - (1 -
+    K/E)^T) + S ceil(T/16), checked against sampled routings), and splits gate/up's K over
     the waves from a larger count; few-expert shapes keep the separate down."""
     from netra_moe.engine import (MERGED_KSPLIT_MIN_TILES, MERGED_MIN_TILES, down_variant,
                                   expected_tiles)
