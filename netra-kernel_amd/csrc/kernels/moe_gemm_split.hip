@@ -35,6 +35,7 @@
 
 #include "moe_ffn_decode.hip"
 #include "moe_numerics.h"
+#include "moe_split_table.h"
 
 #define NK_KERNEL extern "C" __global__
 
@@ -44,103 +45,13 @@ using nk::v4f;
 using nk::v8i;
 using nkstream::lds_barrier;
 
-constexpr uint32_t kMaxE = 513;             // experts, the shared one included
-constexpr uint32_t kPer = (kMaxE + 63) / 64;  // experts per lane of the scan
-
-struct Table {
-  uint32_t n[kMaxE];        // rows of each expert
-  uint32_t off[kMaxE + 1];  // 64-row blocks before it << 16 | chunks before it; [Etot]: all of them
-};
-
-struct Chunk {
-  uint32_t e, row0, tiles, first;  // expert, first sorted row, 16-row tiles, its number among all chunks
-};
-
-// The chunk table, by one wave (the caller puts a barrier behind it). Counts
-// are clamped to T: an operation launched out of order may find another
-// tensor's bytes there.
-template <uint32_t RM>
-__device__ __forceinline__ void build_table(Table& s, const int32_t* __restrict__ counts, uint32_t T, uint32_t Etot,
-                                            uint32_t lane) {
-  const uint32_t per = (Etot + 63u) / 64u;
-  uint32_t n[kPer], c[kPer], b[kPer], cs = 0, bs = 0;
-#pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) {
-    const uint32_t e = lane * per + i;
-    n[i] = (uint32_t)counts[min(e, Etot - 1u)];  // unconditional: all in flight together
-  }
-#pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) n[i] = i < per && lane * per + i < Etot ? min(n[i], T) : 0u;
-#pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) {
-    c[i] = ((n[i] + 15u) / 16u + RM - 1u) / RM;
-    b[i] = (n[i] + 63u) / 64u;
-    cs += c[i];
-    bs += b[i];
-  }
-  uint32_t ci = cs, bi = bs;  // inclusive scans over the lanes
-#pragma unroll
-  for (uint32_t off = 1; off < 64; off <<= 1) {
-    const uint32_t oc = __shfl_up(ci, off), ob = __shfl_up(bi, off);
-    if (lane >= off) { ci += oc; bi += ob; }
-  }
-  if (lane == 63u) s.off[Etot] = bi << 16 | ci;
-  ci -= cs;
-  bi -= bs;
-#pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) {
-    const uint32_t e = lane * per + i;
-    if (i < per && e < Etot) {
-      s.n[e] = n[i];
-      s.off[e] = bi << 16 | ci;
-      ci += c[i];
-      bi += b[i];
-    }
-  }
-}
-
-__device__ __forceinline__ uint32_t all_chunks(const Table& s, uint32_t Etot) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)s.off[Etot]) & 0xffffu;
-}
-
-// Chunk number q (below the total, uniform, every lane active): the last
-// expert whose chunks begin at or before q, by two ballots.
-__device__ __forceinline__ Chunk locate(const Table& s, uint32_t q, uint32_t Etot, uint32_t lane) {
-  const uint32_t per = (Etot + 63u) / 64u;
-  const uint32_t l0 = lane * per;
-  const unsigned long long m0 = __ballot(l0 < Etot && (s.off[min(l0, Etot - 1u)] & 0xffffu) <= q);
-  const uint32_t base = ((uint32_t)__popcll(m0) - 1u) * per;
-  const uint32_t l1 = base + lane;
-  const unsigned long long m1 = __ballot(lane < per && l1 < Etot && (s.off[min(l1, Etot - 1u)] & 0xffffu) <= q);
-  Chunk k;
-  k.e = __builtin_amdgcn_readfirstlane((int)(base + (uint32_t)__popcll(m1) - 1u));
-  const uint32_t off = __builtin_amdgcn_readfirstlane((int)s.off[k.e]), c0 = off & 0xffffu;
-  const uint32_t nc = (__builtin_amdgcn_readfirstlane((int)s.off[k.e + 1u]) & 0xffffu) - c0;
-  const uint32_t tiles = (__builtin_amdgcn_readfirstlane((int)s.n[k.e]) + 15u) / 16u;
-  const uint32_t t0 = (q - c0) * tiles / nc, t1 = (q - c0 + 1u) * tiles / nc;
-  k.row0 = (off >> 16) * 64u + t0 * 16u;
-  k.tiles = t1 - t0;
-  k.first = q;
-  return k;
-}
-
-// This workgroup's share [lo, hi) of `total` positions, workgroups of an XCD
-// (blockIdx % 8) side by side.
-__device__ __forceinline__ void share(uint32_t total, uint32_t& lo, uint32_t& hi) {
-  uint32_t w = blockIdx.x;
-  if (gridDim.x % 8u == 0u) w = (w & 7u) * (gridDim.x / 8u) + (w >> 3);
-  lo = (uint32_t)((uint64_t)w * total / gridDim.x);
-  hi = (uint32_t)((uint64_t)(w + 1u) * total / gridDim.x);
-}
-
 __device__ __forceinline__ float lane_f32(float v, uint32_t l) {
   return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (int)l));
 }
 
 // ---------------------------------------------------------------------------
-// The K blocks are split over SA waves (wave sa: K blocks KBW sa ..), CA =
-// 8 / SA column items side by side, and every wave keeps its K slice of the
-// chunk's activation rows in registers as MFMA operands for as long as the
+// The K blocks are split over the eight waves (wave w: K blocks KBW w ..), and
+// every wave keeps its K slice of the chunk's activation rows in registers as MFMA operands for as long as the
 // workgroup stays on the chunk: an item (16 gate and 16 up rows of W13 over
 // all of K, 64 KiB at H = 2048) is read once, straight into registers, for up
 // to 64 rows, and nothing but weights moves per item. The waves' split sums
@@ -159,13 +70,7 @@ __device__ __forceinline__ float lane_f32(float v, uint32_t l) {
 // branch). Weights are read non-temporally (98 us against 113 with ordinary
 // loads at T = 192).
 constexpr uint32_t kGuWaves = 8;
-constexpr uint32_t RM = 4;    // 16-row tiles per chunk
-constexpr uint32_t kSub = 4;  // row tiles per split-sum buffer
-
-template <uint32_t KB>
-struct GuSplit {
-  static constexpr uint32_t SA = KB < kGuWaves ? KB : kGuWaves, CA = kGuWaves / SA, KBW = KB / SA;
-};
+constexpr uint32_t RM = 4;  // 16-row tiles per chunk
 
 template <uint32_t KBW>
 struct GuBuf {
@@ -178,9 +83,10 @@ __device__ __forceinline__ void gate_up_split(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13,
     const float* __restrict__ w13s, const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ counts,
     uint8_t* __restrict__ hq, float* __restrict__ hs, uint32_t T, uint32_t I, uint32_t Etot, uint32_t cap_blocks) {
-  constexpr uint32_t SA = GuSplit<KB>::SA, CA = GuSplit<KB>::CA, KBW = GuSplit<KB>::KBW;
+  static_assert(KB % kGuWaves == 0, "a whole number of K blocks per wave");
+  constexpr uint32_t KBW = KB / kGuWaves;
   constexpr uint32_t H = 128u * KB;
-  constexpr uint32_t kBufF4 = kGuWaves * 2u * kSub * 64u;  // float4 per split-sum buffer
+  constexpr uint32_t kBufF4 = kGuWaves * 2u * RM * 64u;  // float4 per split-sum buffer
   __shared__ Table s_tab;
   __shared__ __align__(16) float4 s_red[2u * kBufF4];
   constexpr uint32_t kHStride = 128u + 8u;                 // bf16 per LDS h row (+16 bytes rotates banks)
@@ -190,17 +96,17 @@ __device__ __forceinline__ void gate_up_split(
   if (Etot == 0u || Etot > kMaxE) return;  // host-checked
   if (wave == 0) build_table<RM>(s_tab, counts, T, Etot, lane);
   __syncthreads();
-  const uint32_t UP = I / (32u * CA);  // positions per chunk
+  const uint32_t UP = I / 32u;  // positions per chunk
   uint32_t lo, hi;
   // (in whole 128-column blocks of h, which the workgroup requantises)
-  constexpr uint32_t GP = 4u / CA;  // positions per block
+  constexpr uint32_t GP = 4u;  // positions per block
   share(all_chunks(s_tab, Etot) * (UP / GP), lo, hi);
   lo *= GP;
   hi *= GP;
   if (lo >= hi) return;  // uniform
 
-  const uint32_t sa = wave % SA, ca = wave / SA, g4 = lane >> 4;
-  const uint32_t kb0 = sa * KBW;
+  const uint32_t g4 = lane >> 4;
+  const uint32_t kb0 = wave * KBW;
   Chunk ck = locate(s_tab, lo / UP, Etot, lane);
   const uint32_t scale_lane = lane < 2u * KBW ? lane : 0u;
   const uint32_t scale_row = (scale_lane < KBW ? 0u : I / 128u) * KB + kb0 + scale_lane % KBW;
@@ -214,17 +120,23 @@ __device__ __forceinline__ void gate_up_split(
     const float* wse = w13s + (size_t)ck.e * (2u * I / 128u) * KB + scale_row;
     const uint32_t end = min(hi, (ck.first + 1u) * UP);
     GuBuf<KBW> b0, b1;
-    // column item 2 ip + j of the chunk (side by side: CA of them) into a buffer
+    // column item 2 ip + j of the chunk into a buffer (its number opaque: with an
+    // induction variable for every tile's offset a call measured 0.3% more)
+    auto column = [&](uint32_t ip, uint32_t j) __attribute__((always_inline)) {
+      uint32_t c = 2u * ip + j;
+      asm("" : "+s"(c));
+      return c;
+    };
     auto issue_g = [&](GuBuf<KBW>& b, uint32_t ip, uint32_t j, bool live) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t r = nk::buffer_rsrc(we, live ? 2u * I * H : 0u);
-      const uint32_t c = (2u * ip + j) * CA + ca;
+      const uint32_t c = column(ip, j);
       b.ws = wse[(live ? c >> 3 : 0u) * KB];  // (ahead of the tiles it scales)
 #pragma unroll
       for (uint32_t i = 0; i < KBW; ++i) b.g[i] = nk::load_tile_operand<false, true>(r, (2u * c * KB + kb0 + i) * 2048u, lane);
     };
     auto issue_u = [&](GuBuf<KBW>& b, uint32_t ip, uint32_t j, bool live) __attribute__((always_inline)) {
       const __amdgpu_buffer_rsrc_t r = nk::buffer_rsrc(we, live ? 2u * I * H : 0u);
-      const uint32_t c = (2u * ip + j) * CA + ca;
+      const uint32_t c = column(ip, j);
 #pragma unroll
       for (uint32_t i = 0; i < KBW; ++i) b.u[i] = nk::load_tile_operand<false, true>(r, ((2u * c + 1u) * KB + kb0 + i) * 2048u, lane);
     };
@@ -275,79 +187,67 @@ __device__ __forceinline__ void gate_up_split(
           sg[i] = lane_f32(b.ws, i);
           su[i] = lane_f32(b.ws, KBW + i);
         }
+        float4* const red = s_red + par * kBufF4;
+        // two row tiles at a time: their MFMAs are issued back to back and
+        // scaled while the next pair's run (one at a time the chain of MFMA,
+        // scale and LDS write set the time of a many-tile chunk: 140 us for
+        // the shared expert at T = 128, against 85 us for every other share)
+        auto part = [&](const v8i (&w)[KBW], const float (&ws)[KBW], uint32_t gu) __attribute__((always_inline)) {
 #pragma unroll
-        for (uint32_t s0 = 0; s0 < R; s0 += kSub) {
-          constexpr uint32_t kR = R < kSub ? R : kSub;
-          const uint32_t nr = R - s0 < kSub ? R - s0 : kSub;
-          float4* const red = s_red + par * kBufF4;
-          // two row tiles at a time: their MFMAs are issued back to back and
-          // scaled while the next pair's run (one at a time the chain of MFMA,
-          // scale and LDS write set the time of a many-tile chunk: 140 us for
-          // the shared expert at T = 128, against 85 us for every other share)
-          auto part = [&](const v8i (&w)[KBW], const float (&ws)[KBW], uint32_t gu) __attribute__((always_inline)) {
+          for (uint32_t r = 0; r < R; r += 2u) {
+            v4f d[2][KBW];
 #pragma unroll
-            for (uint32_t r = 0; r < kR; r += 2u) {
-              if (r < nr) {
-                v4f d[2][KBW];
+            for (uint32_t h = 0; h < 2u; ++h)
 #pragma unroll
-                for (uint32_t h = 0; h < 2u; ++h)
+              for (uint32_t i = 0; i < KBW; ++i)
+                if (r + h < R) d[h][i] = nk::mfma_e4m3_16x16x128(w[i], a[r + h][i]);
 #pragma unroll
-                  for (uint32_t i = 0; i < KBW; ++i)
-                    if (r + h < nr) d[h][i] = nk::mfma_e4m3_16x16x128(w[i], a[s0 + r + h][i]);
+            for (uint32_t h = 0; h < 2u; ++h) {
+              if (r + h < R) {
+                v4f acc;
 #pragma unroll
-                for (uint32_t h = 0; h < 2u; ++h) {
-                  if (r + h < nr) {
-                    v4f acc;
+                for (uint32_t i = 0; i < KBW; ++i) {
+                  const float s = ws[i] * as[r + h][i];
 #pragma unroll
-                    for (uint32_t i = 0; i < KBW; ++i) {
-                      const float s = ws[i] * as[s0 + r + h][i];
-#pragma unroll
-                      for (uint32_t q = 0; q < 4; ++q) acc[q] = i == 0 ? s * d[h][i][q] : fmaf(s, d[h][i][q], acc[q]);
-                    }
-                    red[((wave * 2u + gu) * kSub + r + h) * 64u + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-                  }
+                  for (uint32_t q = 0; q < 4; ++q) acc[q] = i == 0 ? s * d[h][i][q] : fmaf(s, d[h][i][q], acc[q]);
                 }
+                red[((wave * 2u + gu) * RM + r + h) * 64u + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
               }
             }
-          };
-          part(b.g, sg, 0u);
-          if (s0 + kSub >= R) {
-            __builtin_amdgcn_sched_barrier(0);
-            issue_g(b, p + 1u, j, live);
           }
-          part(b.u, su, 1u);
-          if (s0 + kSub >= R) {
-            __builtin_amdgcn_sched_barrier(0);
-            issue_u(b, p + 1u, j, live);
-          }
-          lds_barrier();  // (the other buffer was read before the previous barrier)
-          // one wave per (column, row tile) adds the SA split sums in order
-          const uint32_t slot = (wave - rot) & (kGuWaves - 1u);
-          if (slot < nr * CA) {
-            const uint32_t r = slot % nr, cs = slot / nr;
-            v4f gs, us;
+        };
+        part(b.g, sg, 0u);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_g(b, p + 1u, j, live);
+        part(b.u, su, 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_u(b, p + 1u, j, live);
+        lds_barrier();  // (the other buffer was read before the previous barrier)
+        // one wave per row tile adds the split sums in order
+        const uint32_t r = (wave - rot) & (kGuWaves - 1u);
+        if (r < R) {
+          v4f gs, us;
 #pragma unroll
-            for (uint32_t w = 0; w < SA; ++w) {
-              const float4 x = red[(((cs * SA + w) * 2u) * kSub + r) * 64u + lane];
-              const float4 y = red[(((cs * SA + w) * 2u + 1u) * kSub + r) * 64u + lane];
-              const v4f xv = {x.x, x.y, x.z, x.w}, yv = {y.x, y.y, y.z, y.w};
+          for (uint32_t w = 0; w < kGuWaves; ++w) {
+            const float4 x = red[((w * 2u) * RM + r) * 64u + lane];
+            const float4 y = red[((w * 2u + 1u) * RM + r) * 64u + lane];
+            const v4f xv = {x.x, x.y, x.z, x.w}, yv = {y.x, y.y, y.z, y.w};
 #pragma unroll
-              for (uint32_t q = 0; q < 4; ++q) {
-                gs[q] = w == 0 ? xv[q] : gs[q] + xv[q];
-                us[q] = w == 0 ? yv[q] : us[q] + yv[q];
-              }
-              // (a few reads in flight: all sixteen would take 64 registers)
-              if (w % 4u == 3u) asm volatile("" : "+v"(gs), "+v"(us) : : "memory");
+            for (uint32_t q = 0; q < 4; ++q) {
+              gs[q] = w == 0 ? xv[q] : gs[q] + xv[q];
+              us[q] = w == 0 ? yv[q] : us[q] + yv[q];
             }
-#pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) us[q] = (kHw ? nk::silu_hw(gs[q]) : nk::silu(gs[q])) * us[q];
-            const uint32_t col = (((2u * p + j) * CA + cs) & 7u) * 16u + g4 * 4u;
-            *reinterpret_cast<uint2*>(&s_h[(r * 16u + (lane & 15u)) * kHStride + col]) =
-                make_uint2(nk::bf16x2_hw(us[0], us[1]), nk::bf16x2_hw(us[2], us[3]));
+            // (a few reads in flight: all sixteen would take 64 registers)
+            if (w % 4u == 3u) asm volatile("" : "+v"(gs), "+v"(us) : : "memory");
           }
-          rot += nr * CA;
-          par ^= 1u;
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) us[q] = (kHw ? nk::silu_hw(gs[q]) : nk::silu(gs[q])) * us[q];
+          const uint32_t col = ((2u * p + j) & 7u) * 16u + g4 * 4u;
+          *reinterpret_cast<uint2*>(&s_h[(r * 16u + (lane & 15u)) * kHStride + col]) =
+              make_uint2(nk::bf16x2_hw(us[0], us[1]), nk::bf16x2_hw(us[2], us[3]));
         }
+        rot += R;
+        par ^= 1u;
       };
       item(b0, 0u);
       item(b1, 1u);

@@ -1,9 +1,11 @@
 """The split gate/up (moe_gemm_split.hip): its dealing of chunks on the CPU,
 and on the GPU the kernel against the path's general kernels and the oracle.
 
-CPU: a restatement of the chunk table and the workgroups' shares covers every
-(16-row tile of an expert, 128-column block of h) exactly once and keeps every
-chunk inside its expert's rows, for drawn and extreme row counts.
+CPU: the kernel's own chunk table and shares (moe_split_table.h, compiled for
+the host) against a restatement of the cut, covering every (16-row tile of an
+expert, 128-column block of h) exactly once and keeping every chunk inside its
+expert's rows, for drawn and extreme row counts and one to nine experts per
+lane.
 
 GPU, at the sizes where a tile count changes (hot: every token on the same
 experts, T rows each): the layer output within the parity bar (2e-2) of the
@@ -12,10 +14,13 @@ inputs: the row scales within one bf16 step (2^-7) and under 1% of the E4M3
 codes different (two fp32 orders of the same sums; the bars of the parity
 tests).
 """
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
-from conftest import gpu_available
+from conftest import REPO, gpu_available
 from netra_moe import engine
 from netra_moe.config import MoEConfig
 
@@ -35,16 +40,34 @@ def chunks_of(counts):
     return out
 
 
-@pytest.mark.parametrize("seed,experts,top", [(0, 257, 13), (1, 257, 70), (2, 513, 5), (3, 24, 416), (4, 1, 1), (5, 33, 64)])
-def test_every_tile_and_column_block_is_dealt_once(seed, experts, top):
+@pytest.fixture(scope="module")
+def host_table(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("split") / "table"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", f"-I{REPO / 'netra-kernel_amd' / 'csrc' / 'kernels'}",
+                    str(Path(__file__).with_name("split_table_host.cpp")), "-o", str(exe)], check=True)
+
+    def run(counts, blocks, T):
+        text = " ".join(map(str, [T, len(counts), RM, GRID, blocks, *counts]))
+        lines = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.split("\n")[:-1]
+        chunks = [tuple(map(int, ln.split())) for ln in lines if not ln.startswith("share")]
+        return chunks, [tuple(map(int, ln.split()[1:])) for ln in lines if ln.startswith("share")]
+
+    return run
+
+
+@pytest.mark.parametrize("seed,experts,top", [(0, 257, 13), (1, 257, 70), (2, 513, 5), (3, 24, 416), (4, 1, 1),
+                                              (5, 33, 64), (6, 513, 416), (7, 64, 17), (8, 65, 129), (9, 512, 1)])
+def test_every_tile_and_column_block_is_dealt_once(seed, experts, top, host_table):
     rng = np.random.default_rng(seed)
     counts = rng.integers(0, top + 1, experts)
     counts[rng.integers(experts)] = top
-    chunks, blocks = chunks_of(counts), 4  # I = 512
-    total = len(chunks) * blocks
+    blocks = 4  # I = 512
+    chunks, shares = host_table(counts, blocks, top)
+    assert chunks == chunks_of(counts)
     seen = np.zeros((sum(-(-n // 64) for n in counts) * 4, blocks), np.int64)
-    for w in range(GRID):
-        for pos in range(w * total // GRID, (w + 1) * total // GRID):
+    for lo, hi in shares:
+        assert hi - lo - len(chunks) * blocks // GRID in (0, 1)
+        for pos in range(lo, hi):
             e, row0, tiles = chunks[pos // blocks]
             assert 1 <= tiles <= RM
             base = 64 * sum(-(-n // 64) for n in counts[:e])
@@ -56,6 +79,11 @@ def test_every_tile_and_column_block_is_dealt_once(seed, experts, top):
         want[4 * block:4 * block + -(-n // 16)] = 1
         block += -(-n // 64)
     np.testing.assert_array_equal(seen, want)
+
+
+def test_counts_beyond_the_tokens_are_clamped(host_table):
+    chunks, _ = host_table([1 << 30, 3], 4, 20)
+    assert chunks == chunks_of([20, 3])
 
 
 @pytest.mark.parametrize("T,E,K,path,split", [(65, 256, 8, "stream", True), (416, 256, 8, "tile", True),
