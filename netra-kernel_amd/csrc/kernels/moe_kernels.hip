@@ -13,12 +13,16 @@
 // a launch; kernels also bound-check data-dependent indices (expert ids,
 // sorted positions) so malformed routing cannot address memory outside the
 // buffers the shapes describe.
+// (The order is the kernels' order in the code object, and it is measured:
+// with the decode kernels right behind the router's, ahead of the prefill front
+// end, the layer takes 36.9 us at T = 5, 72.9 at T = 16 and 98.4 at T = 512,
+// Zipf-skewed (H 2048, I 512, E 256, K 8), against 37.4, 73.5 and 99.6 with the
+// same kernels behind it; which of the prefill parts comes first makes 0.5%.)
 #include "moe_router.hip"
-#include "moe_route_prefill.hip"
 #include "moe_gemm_stream.hip"
-#include "moe_ffn_decode.hip"
+#include "moe_ffn_decode.hip"  // (and moe_gemm_lds.hip)
 #include "moe_gemm_split.hip"
 #include "moe_gemm_tile.hip"
-#include "moe_gemm_lds.hip"
+#include "moe_route_prefill.hip"
 #include "moe_misc.hip"
 #include "moe_bridge_kernels.hip"
