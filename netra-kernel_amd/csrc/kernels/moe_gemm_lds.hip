@@ -165,17 +165,17 @@ __device__ __forceinline__ bool xcd_item(uint32_t i, uint32_t n, uint32_t& item)
 // tile16x128 layout; the copies move the same 2 KiB blocks, only the up tile's
 // place and the operand reads out of LDS differ.
 // kChoose: an item whose expert has no other block pair (a tail that it
-// absorbs is not one) copies W13 with non-temporal loads (no other item reads
-// that slice, and its lines leave the activations in the L2); with more pairs
-// the copies are ordinary, and the pairs' items find each other's lines
-// there. gate/up us at H 2048, I 512, E 256, K 8, all ordinary / all
-// non-temporal / chosen: T = 512 113.1 / 107.0 / 106.0, 1000 115.9 / 110.9 /
-// 108.9, 2048 121.7 / 119.6 / 119.1, 4096 145.4 / 149.8 / 145.4; Zipf-skewed
-// 512 46.2 / 43.3 / 41.1, 1000 60.8 / 61.0 / 56.9, 4096 140.1 / 147.7 / 137.2.
-// The K loop is there once for each kind of copy: a branch in every copy
-// measured 62.7 against 60.4 (Zipf T = 1000). (H 1024, whose tens of MB of
-// weights the caches hold: 39.4 / 44.2 at T = 2000, E 24, so only H 2048 has
-// the choice.)
+// absorbs is not one) copies W13 with non-temporal loads, since no other item
+// reads that slice; with more pairs the copies are ordinary, and the pairs'
+// items find each other's lines in the L2. gate/up us at H 2048, I 512, E 256,
+// K 8, all ordinary / all non-temporal / chosen: T = 512 113.1 / 107.0 / 106.0,
+// 1000 115.9 / 110.9 / 108.9, 2048 121.7 / 119.6 / 119.1, 4096 145.4 / 149.8 /
+// 145.4; Zipf-skewed 512 46.2 / 43.3 / 41.1, 1000 60.8 / 61.0 / 56.9, 4096
+// 140.1 / 147.7 / 137.2. (Few of the bytes: it fetches 552 MB against 559 at T =
+// 1000, 199 against 205 at T = 512, skewed.) The K loop is there once for each
+// kind of copy: a branch in every copy measured 62.7 against 60.4 (Zipf T =
+// 1000). (H 1024, whose tens of MB of weights the caches hold: 39.4 / 44.2 at T
+// = 2000, E 24, so only H 2048 has the choice.)
 template <uint32_t KB, bool kAiter = false, bool kChoose = false>  // H / 128
 __device__ __forceinline__ void gate_up_lds(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w13,
