@@ -1,7 +1,7 @@
 """Static checks of the built gfx950 code object for what the compiler
 cannot see around inline assembly:
 
-* a vector-memory instruction (buffer/global/flat) that reads an SGPR fewer
+* a vector-memory instruction (buffer/global/flat/scratch) that reads an SGPR fewer
   than five wait states after a VALU instruction wrote it (v_readfirstlane,
   v_readlane, VALU compares and carry-outs). The hardware needs those wait
   states; the compiler inserts them for its own instructions but not around
@@ -39,7 +39,7 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 WAIT_STATES = 5
 
 _SREG = re.compile(r"\bs\[(\d+):(\d+)\]|\bs(\d+)\b|\b(vcc|exec|m0)\b")
-_VMEM = re.compile(r"^(buffer_|global_|flat_)")
+_VMEM = re.compile(r"^(buffer_|global_|flat_|scratch_)")
 
 
 def sgprs(text: str) -> set:
@@ -153,7 +153,7 @@ def test_no_valu_sgpr_to_vmem_hazard_in_any_kernel(artefact):
 RING_WAITS = {"netra_moe_gate_up_lds_": {0, 6, 7}, "netra_moe_route_screen_": {0, 8, 16}}
 KCOPIES = 7
 _VMCNT = re.compile(r"vmcnt\((\d+)\)")
-_VSTORE = re.compile(r"(global|buffer|flat)_store")
+_VSTORE = re.compile(r"(global|buffer|flat|scratch)_store")
 
 
 def ring_violations(lines: list[str], waits: set[int] | None = None) -> list[str]:
