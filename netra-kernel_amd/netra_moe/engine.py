@@ -24,6 +24,7 @@ import json
 import math
 import shutil
 from dataclasses import dataclass
+from functools import lru_cache
 from pathlib import Path
 
 from .config import BLOCK_M, MoEConfig
@@ -526,12 +527,20 @@ MERGED_MIN_TILES = {(512, 256): 0, (2048, 512): 128}
 MERGED_KSPLIT_MIN_TILES = {(2048, 512): 150}
 
 
+@lru_cache(maxsize=1024)  # (an engine's compilation asks some thirty times; 40 us each)
+def _tiles_per_expert(T: int, E: int, K: int) -> float:
+    """16-row tiles a routed expert is expected to have: rows binomial (T, K / E)."""
+    if K == E:
+        return float((T + 15) // 16)
+    lp, lq, lt = math.log(K / E), math.log1p(-K / E), math.lgamma(T + 1)  # (in logs: T may be thousands)
+    return sum(math.exp(lt - math.lgamma(n + 1) - math.lgamma(T - n + 1) + n * lp + (T - n) * lq) * ((n + 15) // 16)
+               for n in range(1, T + 1))
+
+
 def expected_tiles(cfg: MoEConfig) -> float:
-    """16-row tiles of a decode call under uniform routing: each routed expert's
-    rows, binomial (T, K / E), in tiles of 16, plus the shared experts' tiles."""
-    T, p = cfg.T, cfg.K / cfg.E
-    routed = sum(math.comb(T, n) * p ** n * (1.0 - p) ** (T - n) * ((n + 15) // 16) for n in range(1, T + 1))
-    return cfg.E * routed + cfg.S * ((T + 15) // 16)
+    """16-row tiles of a decode call under uniform routing: the routed experts',
+    every one of each, plus the shared experts'."""
+    return cfg.E * _tiles_per_expert(cfg.T, cfg.E, cfg.K) + cfg.S * ((cfg.T + 15) // 16)
 
 
 def down_variant(cfg: MoEConfig) -> str:

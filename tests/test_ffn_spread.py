@@ -40,7 +40,8 @@ def test_columns_per_workgroup(shape, P):
     assert ("gate_up_down" in sym) or sym.endswith("_wide_gfx950" if P == full else f"_wide_p{P}_gfx950")
 
 
-@pytest.mark.parametrize("T,E,K,S", [(64, 16, 8, 1), (64, 24, 8, 1), (40, 24, 8, 0), (64, 32, 15, 1), (17, 16, 2, 1)])
+@pytest.mark.parametrize("T,E,K,S", [(64, 16, 8, 1), (64, 24, 8, 1), (40, 24, 8, 0), (64, 32, 15, 1), (17, 16, 2, 1),
+                                     (64, 8, 8, 1), (3000, 16, 4, 1)])
 def test_expected_tiles_counts_every_tile_of_an_expert(T, E, K, S):
     rng = np.random.default_rng(T * E + K)
     counts = np.stack([np.bincount(np.argsort(rng.random((T, E)), axis=1)[:, :K].ravel(), minlength=E)
